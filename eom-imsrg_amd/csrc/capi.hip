@@ -121,6 +121,12 @@ struct imsrg_basis_s {
   Partner* partT = nullptr;
   int pstride = 0;
   int *rowp = nullptr, *colp = nullptr;
+  // 122 by closed tiles (t122_ok: every closed set fits a tile)
+  bool t122_ok = false;
+  T122Plan t122{};
+  TaskList<T122Task> t122t;
+  std::vector<int> t122_rent, t122_rcnt, t122_cent, t122_ccnt;
+  std::vector<int2> t122_rrec, t122_crec;
   std::vector<QuadItem> quad_h;   // 222_ph outputs, quadruple-major (grouped path)
   QuadItem* quad = nullptr;
   // the same outputs in chunks of quadruples (k_comm222ph_chunk)
@@ -336,6 +342,109 @@ int family_tasks(imsrg_basis_s* B, GemmFamily& f, int tile) {
   return rc;
 }
 
+// the closed tiles of 122 (T122Plan) from the partner lists of build_plan
+void build_t122(imsrg_basis_s* B, const std::vector<int>& order) {
+  const Basis& b = B->b;
+  B->t122_ok = false;
+  B->t122t.host.clear();
+  B->t122t.chan_begin.assign(1, 0);
+  for (std::vector<int>* v : {&B->t122_rent, &B->t122_rcnt, &B->t122_cent, &B->t122_ccnt}) v->clear();
+  T122Plan& P = B->t122;
+  P = T122Plan{};
+  struct Set { int a, b; std::vector<int> ent; };   // one pair of (l, j, tz) blocks
+  struct Group { int row0, nrow; std::vector<std::pair<int, int>> slab; };   // (col0, ncol)
+  std::vector<std::vector<Set>> sets(b.nblocks);
+  int big = 0;
+  for (int q = 0; q < b.nblocks; ++q) {
+    std::map<std::pair<int, int>, std::vector<int>> m;
+    for (int c = 0; c < 3; ++c)
+      for (int ix = 0; ix < b.dims[q * 3 + c]; ++ix) {
+        const int x = b.spblk[b.pl[q * 3 + c][2 * ix]], y = b.spblk[b.pl[q * 3 + c][2 * ix + 1]];
+        m[{std::min(x, y), std::max(x, y)}].push_back((c << 28) | ix);
+      }
+    for (auto& kv : m) {
+      big = std::max(big, (int)kv.second.size());
+      sets[q].push_back(Set{kv.first.first, kv.first.second, std::move(kv.second)});
+    }
+  }
+  // slabs as wide as the kernels' unrolled column counts
+  if (big > kT122Cols) return;
+  const int cap = big <= 16 ? 16 : (big <= 32 ? 32 : (big <= 40 ? 40 : kT122Cols));
+  auto emit = [&](int q, std::vector<int> ent, const std::vector<int>& ptr, std::vector<int>& out,
+                  std::vector<int>& cnt, std::vector<std::vector<int2>>& recs) {
+    std::sort(ent.begin(), ent.end());
+    std::map<int, int> at;
+    for (size_t x = 0; x < ent.size(); ++x) at[ent[x]] = (int)x;
+    for (int e : ent) {
+      const int c = e >> 28, ix = e & 0xfffffff;
+      const size_t gid = (size_t)b.pairoff[q * 3 + c] + ix;
+      const bool same = b.pl[q * 3 + c][2 * ix] == b.pl[q * 3 + c][2 * ix + 1];
+      std::vector<int2> r;
+      for (int k = ptr[gid]; k < ptr[gid + 1]; ++k) {
+        const Partner& p = B->part_h[k];
+        const auto it = at.find((((p.code >> 22) & 3) << 28) | (p.code & 0x3fffff));
+        if (it == at.end()) return false;
+        const int s2 = (p.code >> 26) & 1;
+        r.push_back(int2{it->second | (((p.code >> 24) & 1) << 17) | (((p.code >> 25) & 1) << 18) |
+                             ((s2 == (same ? 1 : 0) ? 0 : (s2 ? 1 : 2)) << 19),
+                         B->f1off_h[p.fk]});
+      }
+      if (r.size() > (size_t)kT122Recs) return false;
+      P.maxrec = std::max(P.maxrec, (int)r.size());
+      out.push_back(e);
+      cnt.push_back((int)r.size());
+      recs.push_back(std::move(r));
+    }
+    return true;
+  };
+  std::vector<std::vector<int2>> rr, cr;
+  for (int q : order) {
+    std::vector<Group> gs;
+    size_t x = 0;
+    while (x < sets[q].size()) {
+      size_t e = x;
+      int n = 0;
+      while (e < sets[q].size() && n + (int)sets[q][e].ent.size() <= kT122Rows) n += (int)sets[q][e++].ent.size();
+      Group g{(int)B->t122_rent.size(), n, {}};
+      std::vector<int> ent;
+      for (size_t y = x; y < e; ++y) ent.insert(ent.end(), sets[q][y].ent.begin(), sets[q][y].ent.end());
+      if (!emit(q, ent, B->rowp_h, B->t122_rent, B->t122_rcnt, rr)) return;
+      for (size_t y = x; y < e;) {
+        std::vector<int> ce;
+        const int c0 = (int)B->t122_cent.size();
+        while (y < e && ce.size() + sets[q][y].ent.size() <= (size_t)cap) {
+          ce.insert(ce.end(), sets[q][y].ent.begin(), sets[q][y].ent.end());
+          ++y;
+        }
+        if (!emit(q, ce, B->colp_h, B->t122_cent, B->t122_ccnt, cr)) return;
+        g.slab.push_back({c0, (int)ce.size()});
+        P.maxcol = std::max(P.maxcol, (int)ce.size());
+      }
+      gs.push_back(std::move(g));
+      x = e;
+    }
+    // the row groups against one slab side by side: their elements share
+    // columns
+    for (size_t gb = 0; gb < gs.size(); ++gb)
+      for (const auto& sl : gs[gb].slab)
+        for (size_t ga = 0; ga <= gb; ++ga)
+          B->t122t.host.push_back(T122Task{q, gs[ga].row0, gs[ga].nrow, sl.first, sl.second, ga == gb ? 1 : 0, 0, 0});
+    B->t122t.chan_begin.push_back((int)B->t122t.host.size());
+  }
+  P.nrows = (int)B->t122_rent.size();
+  P.ncols = (int)B->t122_cent.size();
+  if (P.maxrec < 1) P.maxrec = 1;
+  auto flat = [](const std::vector<std::vector<int2>>& v, int maxrec, std::vector<int2>& out) {
+    out.assign((size_t)maxrec * v.size(), int2{0, 0});
+    for (size_t i = 0; i < v.size(); ++i)
+      for (size_t k = 0; k < v[i].size(); ++k) out[k * v.size() + i] = v[i][k];
+  };
+  flat(rr, P.maxrec, B->t122_rrec);
+  flat(cr, P.maxrec, B->t122_crec);
+  B->t122t.n = (int)B->t122t.host.size();
+  B->t122_ok = B->t122t.n >= kT122MinTiles;
+}
+
 int build_plan(imsrg_basis_s* B) {
   const Basis& b = B->b;
   const std::vector<int> order = channel_order(b);
@@ -544,6 +653,7 @@ int build_plan(imsrg_basis_s* B) {
       for (int k = 0; k < B->rowp_h[gi + 1] - B->rowp_h[gi]; ++k)
         B->partT_h[(size_t)k * npairs + gi] = B->part_h[B->rowp_h[gi] + k];
   }
+  build_t122(B, order);
   // 222_ph outputs as (orbit quadruple, 2J) items, J fastest: every upper
   // element of every channel exactly once (checked against seg_tri)
   {
@@ -688,6 +798,13 @@ int build_plan(imsrg_basis_s* B) {
     return rc;
   if ((rc = upload(B, B->part_h, &B->partners))) return rc;
   if ((rc = upload(B, B->partT_h, &B->partT))) return rc;
+  if (B->t122_ok) {
+    if ((rc = upload(B, B->t122_rent, (int**)&B->t122.rent)) || (rc = upload(B, B->t122_rcnt, (int**)&B->t122.rcnt)) ||
+        (rc = upload(B, B->t122_rrec, (int2**)&B->t122.rrec)) || (rc = upload(B, B->t122_cent, (int**)&B->t122.cent)) ||
+        (rc = upload(B, B->t122_ccnt, (int**)&B->t122.ccnt)) || (rc = upload(B, B->t122_crec, (int2**)&B->t122.crec)) ||
+        (rc = upload(B, B->t122t.host, &B->t122t.dev)))
+      return rc;
+  }
   if ((rc = upload(B, B->f1off_h, &B->f1off))) return rc;
   if ((rc = upload(B, B->rowp_h, &B->rowp))) return rc;
   if ((rc = upload(B, B->colp_h, &B->colp))) return rc;
@@ -817,6 +934,12 @@ void t_121(const Exec& X, const double* L, int Lh, const double* R, int Rh, doub
 void t_122(const Exec& X, const double* L, int Lh, const double* R, int Rh, double* RES, int RESh,
            hipStream_t s, bool mirror = true) {
   imsrg_basis_s* B = X.B;
+  if (B->t122_ok) {
+    run(B, B->t122t, [&](const T122Task* t, int n) {
+      launch_comm122t(X.D, B->t122, t, n, L, Lh, R, Rh, RES, RESh, s, mirror ? 1 : 0);
+    });
+    return;
+  }
   run(B, B->seg_tri, [&](const SegTask* t, int n) {
     launch_comm122p(X.D, t, n, B->partners, B->partT, B->pstride, B->rowp, B->colp, B->f1off, B->nf1, L, Lh, R, Rh,
                     RES, RESh, s,

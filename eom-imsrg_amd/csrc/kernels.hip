@@ -143,6 +143,248 @@ void launch_comm122p(const DevBasis& B, const SegTask* t, int nt, const Partner*
                      pstride, rowp, colp, f1off, nf1, L, Lh, R, Rh, RES, RESh, mirror);
 }
 
+// ---------------------------------------------- commutator_122 by closed tiles
+// One workgroup per tile (row group x column slab, see T122Plan) of one
+// channel.  The tile of both operands is staged in LDS as full-matrix elements
+// M(r, c) (herm applied to elements stored transposed), so each stored
+// element is read from memory once, along contiguous runs of the ordered row
+// entries; the partner sums
+//   RES(r, c) = sum_k FL(r, k) R(k, c) - FR(r, k) L(k, c)
+//             - sum_k R(r, k) GL(k, c) - L(r, k) GR(k, c)
+// then read LDS only.  Lanes hold the rows (their records' coefficients in
+// registers), waves take the columns (their records broadcast from LDS).
+// Tiles cover every unordered pair of groups once: off the diagonal the
+// elements of (column, row) follow from RES(c, r) = -Lh Rh RES(r, c) and are
+// written through LDS along the columns, so both orientations are stored in
+// contiguous runs.  mirror = 0: only the upper triangles of the square blocks.
+// The list kernel above is bound by the address path (about 42 vector loads an
+// element); here an element costs two loads, one store and about 30 LDS reads.
+// What bounds it now is the chain of a tile (entries, records, coefficients,
+// elements, sums: waves wait 56 % of their cycles at four a SIMD) and, at eMax
+// 10, HBM: 850 MB in 404 us.  Upper triangles, eMax 6 / 8 / 10: 15.3 / 64 / 404
+// us against 17.5 / 128 / 892 us by lists.  Tried and slower: several slabs a
+// workgroup (the addresses kept across slabs spill), one wave's own copy of
+// the row coefficients (12 dependent loads a lane), the columns as the outer
+// loop of the row sums (a branch per record and column).
+// coefficient of a record for one operand's one-body element f: its sign and
+// sqrt 2 factor, and the herm factor of an element read transposed
+__device__ __forceinline__ double t122_coef(int rec, double f, int neg_tr) {
+  const int k = (rec >> 19) & 3;
+  const double a = k == 0 ? f : f * (k == 1 ? 1.4142135623730951 : 0.70710678118654757);
+  return (((rec >> 18) & 1) ^ (((rec >> 17) & 1) & neg_tr)) ? -a : a;
+}
+
+// MAXR: records of a row held in registers; NJ: columns of a wave (4 NJ >= slab)
+template <int MAXR, int NJ>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NJ <= 8 ? 4 : 3))) void k_comm122t(
+    DevBasis B, T122Plan P, const T122Task* tasks, const double* L, int Lh, const double* R, int Rh, double* RES,
+    int RESh, int mirror) {
+  int inst;
+  if (!batch_inst(B, inst)) return;
+  L += (i64)inst * B.oplen;
+  R += (i64)inst * B.oplen;
+  RES += (i64)inst * B.oplen;
+  // (row r, column c) of the tiles at c * LD + r: compile-time strides, so the
+  // columns of a wave are immediate offsets of one address per record; the
+  // padding row kT122Rows holds zeros, read by the lanes with fewer records
+  constexpr int LD = kT122Rows + 1, NC = 4 * NJ;
+  static_assert(2 * MAXR * kT122Rows <= 2 * NC * LD, "the row coefficients pass through the tiles' LDS");
+  __shared__ double tile[2 * NC * LD];
+  __shared__ double cf[2 * NC * MAXR];   // column coefficients (gL, gR) of record k of column c
+  __shared__ int cl[NC * MAXR];          // their column offsets in the tile
+  double* const tL = tile;
+  double* const tR = tile + NC * LD;
+  const T122Task t = tasks[xcd_contig(blockIdx.x, gridDim.x)];   // neighbouring tiles share lines
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lneg = Lh < 0, rneg = Rh < 0;
+  const int nrow = t.nrow;
+  const i64* go = B.goff + t.q * 6;
+  const int d0 = B.dims[t.q * 3], d1 = B.dims[t.q * 3 + 1], d2 = B.dims[t.q * 3 + 2];
+  const i64 g0 = go[0], g11 = go[3], g22 = go[4], x12 = go[5] - go[3];
+  const bool rok = lane < nrow;
+  const int re = rok ? P.rent[t.row0 + lane] : 0;
+  const int nr = rok ? P.rcnt[t.row0 + lane] : 0;
+  const int rcls = re >> 28, ridx = re & 0xfffffff;
+  const int ldr = pick3(rcls, d0, d1, d2);
+  // Stored position of (row, column of class cc and index ic), row class <=
+  // cc: the blocks of row class pp are one matrix of d0 rows over all columns
+  // (p0 = the column's place there); class ph has two blocks, hh one.
+  const i64 rbase = (rcls == 0 ? g0 : (rcls == 1 ? g11 : g22)) + ridx;
+  auto at = [&](int cc, int ic, int p0) -> i64 {
+    return rbase + (i64)(rcls == 0 ? p0 : ic) * ldr + (rcls == 1 && cc == 2 ? x12 : 0);
+  };
+  const int np = __popcll(__ballot(rok && rcls == 0));   // rows of class pp (the entries are ordered by class)
+  int nmax = nr;   // most records of a row
+  for (int o = 32; o > 0; o >>= 1) nmax = max(nmax, __shfl_xor(nmax, o, 64));
+  nmax = __builtin_amdgcn_readfirstlane(nmax);
+  const int hnat = -Lh * Rh;
+  double fl[MAXR], fr[MAXR];
+  int rl[MAXR];
+  const int ncol = t.ncol;
+  const bool cok = lane < ncol;
+  // column entries and record counts, column c in lane c of every wave
+  const int ce_l = cok ? P.cent[t.col0 + lane] : 0;
+  const int cn_l = cok ? P.ccnt[t.col0 + lane] : 0;
+  const int ccls_l = ce_l >> 28, cidx_l = ce_l & 0xfffffff;
+  const int p0_l = cidx_l + pick3(ccls_l, 0, d0, d0 + d1);
+  // elements stored as (r, c), lanes along the rows, into registers
+  double pl[NJ], pr[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const int c = wave + 4 * j;
+    pl[j] = pr[j] = 0.0;
+    if (c < ncol) {
+      const int ce = __builtin_amdgcn_readlane(ce_l, c), p0 = __builtin_amdgcn_readlane(p0_l, c);
+      if (rok && rcls <= (ce >> 28)) {
+        const i64 o = at(ce >> 28, ce & 0xfffffff, p0);
+        pl[j] = L[o];
+        pr[j] = R[o];
+      }
+    }
+  }
+  // column coefficients
+  for (int x = tid; x < ncol * MAXR; x += 256) {
+    const int c = x / MAXR, k = x - c * MAXR;
+    if (k < P.ccnt[t.col0 + c]) {
+      const int2 rec = P.crec[(i64)k * P.ncols + t.col0 + c];
+      cf[2 * x] = t122_coef(rec.x, L[rec.y], lneg);
+      cf[2 * x + 1] = t122_coef(rec.x, R[rec.y], rneg);
+      cl[x] = (rec.x & 63) * LD;
+    }
+  }
+  // row coefficients, formed once by the workgroup and kept in every
+  // wave's registers
+  {
+    for (int x = tid; x < nmax * kT122Rows; x += 256) {
+      const int r = x & (kT122Rows - 1), k = x / kT122Rows;   // this lane's own row
+      double vl = 0.0, vr = 0.0;
+      if (k < nr) {
+        const int2 rec = P.rrec[(i64)k * P.nrows + t.row0 + r];
+        vl = t122_coef(rec.x, L[rec.y], lneg);
+        vr = t122_coef(rec.x, R[rec.y], rneg);
+      }
+      tile[2 * x] = vl;
+      tile[2 * x + 1] = vr;
+    }
+#pragma unroll
+    for (int k = 0; k < MAXR; ++k)
+      rl[k] = wave * LD + (k < nr ? (P.rrec[(i64)k * P.nrows + t.row0 + lane].x & 63) : kT122Rows);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < MAXR; ++k)
+      if (k < nmax) {
+        fl[k] = tile[2 * (k * kT122Rows + lane)];
+        fr[k] = tile[2 * (k * kT122Rows + lane) + 1];
+      }
+    __syncthreads();
+  }
+  if (tid < NC) tL[tid * LD + kT122Rows] = tR[tid * LD + kT122Rows] = 0.0;
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const int c = wave + 4 * j;
+    if (c < ncol && rok && rcls <= (__builtin_amdgcn_readlane(ce_l, c) >> 28)) {
+      tL[c * LD + lane] = pl[j];
+      tR[c * LD + lane] = pr[j];
+    }
+  }
+  // elements stored as (c, r), class of c below the class of r: lanes along
+  // the columns
+  const i64 cbase = (ccls_l == 0 ? g0 : (ccls_l == 1 ? g11 : g22)) + cidx_l;
+  const int ldc = pick3(ccls_l, d0, d1, d2);
+  auto atc = [&](int kr, int ir) -> i64 {
+    return cbase + (i64)(ccls_l == 0 ? ir + pick3(kr, 0, d0, d0 + d1) : ir) * ldc + (ccls_l == 1 && kr == 2 ? x12 : 0);
+  };
+#pragma unroll 4
+  for (int r = np + wave; r < nrow; r += 4) {
+    const int er = __builtin_amdgcn_readlane(re, r);
+    const int kr = er >> 28;
+    if (cok && ccls_l < kr) {
+      const i64 o = atc(kr, er & 0xfffffff);
+      tL[lane * LD + r] = Lh * L[o];
+      tR[lane * LD + r] = Rh * R[o];
+    }
+  }
+  __syncthreads();
+  // this lane's outputs of columns wave, wave + 4, ... (those past the slab
+  // sum whatever the tile holds and are not stored)
+  double val[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) val[j] = 0.0;
+#pragma unroll
+  for (int k = 0; k < MAXR; ++k)
+    if (k < nmax) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        val[j] = fma(fl[k], tR[rl[k] + 4 * j * LD], val[j]);
+        val[j] = fma(-fr[k], tL[rl[k] + 4 * j * LD], val[j]);
+      }
+    }
+  const int row = rok ? lane : kT122Rows;
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const int c = wave + 4 * j;
+    if (c < ncol) {
+      const int nk = __builtin_amdgcn_readlane(cn_l, c);
+      const int* clc = cl + c * MAXR;
+      const double* cfc = cf + 2 * c * MAXR;
+#pragma unroll 2
+      for (int k = 0; k < nk; ++k) {
+        const int o = clc[k] + row;
+        val[j] = fma(-cfc[2 * k], tR[o], val[j]);
+        val[j] = fma(cfc[2 * k + 1], tL[o], val[j]);
+      }
+    }
+  }
+  // outputs stored as (r, c)
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const int c = wave + 4 * j;
+    if (c < ncol) {
+      const int ce = __builtin_amdgcn_readlane(ce_l, c), p0 = __builtin_amdgcn_readlane(p0_l, c);
+      const int cc = ce >> 28, ic = ce & 0xfffffff;
+      // kept: every class pair below the diagonal, the upper triangle and,
+      // with mirror, the lower one of the square blocks
+      if (rok && (rcls < cc || (rcls == cc && (mirror || ridx <= ic))))
+        RES[at(cc, ic, p0)] =
+            rcls < cc || ridx < ic ? val[j] : (ridx == ic ? (mirror ? val[j] * RESh : val[j]) : val[j] * (hnat * RESh));
+    }
+  }
+  if (t.diag) return;
+  // the other orientation, through LDS: lanes along the columns
+  __syncthreads();
+  {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int c = wave + 4 * j;
+      if (c < ncol && rok) tL[c * LD + lane] = val[j];
+    }
+    __syncthreads();
+#pragma unroll 2
+    for (int r = wave; r < nrow; r += 4) {
+      const int er = __builtin_amdgcn_readlane(re, r);
+      const int kr = er >> 28, ir = er & 0xfffffff;
+      if (cok && (ccls_l < kr || (ccls_l == kr && (mirror || cidx_l < ir)))) {
+        const double v = tL[lane * LD + r];
+        RES[atc(kr, ir)] = v * (ccls_l < kr || cidx_l < ir ? hnat : RESh);
+      }
+    }
+  }
+}
+
+void launch_comm122t(const DevBasis& B, const T122Plan& P, const T122Task* t, int nt, const double* L, int Lh,
+                     const double* R, int Rh, double* RES, int RESh, hipStream_t s, int mirror) {
+  if (nt <= 0) return;
+  const dim3 g(nt, B.ninst), w(256);
+#define IMSRG_122T(MR, NJ) \
+  hipLaunchKernelGGL((k_comm122t<MR, NJ>), g, w, 0, s, B, P, t, L, Lh, R, Rh, RES, RESh, mirror)
+  // blocks of n orbits have n^2 columns and 2 n records: n <= 4, 5, 6, 7
+  if (P.maxrec <= 8 && P.maxcol <= 16) IMSRG_122T(8, 4);
+  else if (P.maxrec <= 10 && P.maxcol <= 32) IMSRG_122T(10, 8);
+  else if (P.maxrec <= 12 && P.maxcol <= 40) IMSRG_122T(12, 10);
+  else IMSRG_122T(16, 14);
+#undef IMSRG_122T
+}
+
 // ================================================== commutator_222_ph scatter
 // commutators.f90:804-923.  Every J' term of the reference reads WCC and
 // its transpose only in the combination

@@ -32,6 +32,37 @@ struct QuadItem { int ijkl; int J; };
 struct Partner { int code; int fk; };
 constexpr int kF1Max = 2048;   // compact one-body elements of the 122 partner sums
 
+// commutator_122 by closed tiles (k_comm122t).  The partner sums of a pair
+// (a, b) replace one orbit inside its (l, j, tz) block, so the pairs of one
+// pair of (l, j, tz) blocks only ever read each other.  Every channel's pairs
+// (all three classes) are cut into groups of at most kT122Rows such closed
+// sets, ordered by (class, index); a slab is a closed subset of a group used
+// as tile columns.  Entries: class << 28 | index in the class list.
+// Records: x = local partner index | f transposed << 17 | negative << 18 |
+// factor << 19 (0: 1, 1: sqrt 2, 2: 1 / sqrt 2), y = operator offset of the
+// one-body element.
+constexpr int kT122Rows = 64;
+constexpr int kT122Cols = 56;     // most slab columns
+constexpr int kT122Recs = 16;     // most records of one pair
+// From three tiles per CU on (what a CU holds at once): below, the chip is not
+// full and the tile's longer chain (records, coefficients, tile, sums) shows:
+// eMax 5 (354 tiles) 12.5 us against 8.2 us by lists; eMax 6 (912) 15.3
+// against 17.5, eMax 8 (2976) 64 against 128, eMax 10 (12104) 404 against 892.
+constexpr int kT122MinTiles = 768;
+// row group [row0, row0 + nrow) against the slab [col0, col0 + ncol); diag:
+// the slab belongs to the row group itself
+struct T122Task { int q; int row0, nrow; int col0, ncol; int diag; int pad0, pad1; };
+struct T122Plan {
+  const int* rent;      // [nrows] row entries, group after group
+  const int* rcnt;      // [nrows] records of each
+  const int2* rrec;     // [maxrec * nrows] record k of entry x at k * nrows + x
+  const int* cent;      // [ncols] column entries, slab after slab
+  const int* ccnt;
+  const int2* crec;     // [maxrec * ncols]
+  int nrows, ncols;
+  int maxcol, maxrec;   // largest slab, most records of a pair
+};
+
 // Tile of up to kTile CCX elements of cross-coupled block q1
 struct CCTask { int q1; int start; };
 
@@ -138,6 +169,9 @@ void launch_hf_unpack(const DevBasis& B, const SegTask* t, int nt, const double*
 void launch_comm122p(const DevBasis& B, const SegTask* t, int nt, const Partner* part, const Partner* partT,
                      int pstride, const int* rowp, const int* colp, const int* f1off, int nf1, const double* L, int Lh,
                      const double* R, int Rh, double* RES, int RESh, hipStream_t s, int mirror = 1);
+// the same by closed tiles
+void launch_comm122t(const DevBasis& B, const T122Plan& P, const T122Task* t, int nt, const double* L, int Lh,
+                     const double* R, int Rh, double* RES, int RESh, hipStream_t s, int mirror);
 void launch_pandya(const DevBasis& B, const CCTask* t, int nt, const double* op, int herm, double* CC,
                    hipStream_t s);
 void launch_comm111(const DevBasis& B, const double* L, int Lh, const double* R, int Rh, double* RES,
