@@ -134,6 +134,12 @@ struct imsrg_basis_s {
   std::vector<int> fq_h, fql_h, fqi_h;
   PhChunk* phc = nullptr;
   int *fq = nullptr, *fql = nullptr, *fqi = nullptr;
+  // 222_ph by block quadruples (phb_ok: every quadruple fits a chunk)
+  bool phb_ok = false;
+  PhbPlan phbp{};
+  std::vector<PhbQuad> phbq_h;
+  std::vector<PhbSlot> phbs_h;
+  std::vector<int> phb_rows_h, phb_mem_h;
   std::vector<OneTask> one_h;
   OneTask* one = nullptr;
   // norm chunks
@@ -445,6 +451,120 @@ void build_t122(imsrg_basis_s* B, const std::vector<int>& order) {
   B->t122_ok = B->t122t.n >= kT122MinTiles;
 }
 
+// 222_ph by block quadruples: the cross-coupled rows in block order, the
+// quadruples and their slots (PhbPlan)
+void build_phb(imsrg_basis_s* B) {
+  const Basis& b = B->b;
+  B->phb_ok = false;
+  B->phbq_h.clear(); B->phbs_h.clear(); B->phb_mem_h.clear();
+  for (int o : b.spmem) B->phb_mem_h.push_back(o | (b.con[o] << 8));
+  const int nb = (int)b.spstart.size() - 1, N = b.N;
+  auto size = [&](int A) { return b.spstart[A + 1] - b.spstart[A]; };   // a block may be empty
+  for (int A = 0; A < nb; ++A)
+    if (size(A) > kPhbMembers) return;
+  // rows of every cross-coupled block sorted by (block of a, block of b, a, b)
+  std::vector<int> rowbase((size_t)b.nJ * nb * nb, -1);
+  B->phb_rows_h.assign(b.ccrows.size(), 0);
+  for (int h = 0; h < b.nJ; ++h)
+    for (int T = 0; T <= 1; ++T)
+      for (int P = 0; P <= 1; ++P) {
+        const int q = h + T * (b.JTM + 1) + 2 * P * (b.JTM + 1);
+        if (q >= b.ncc) continue;
+        int at = 0;
+        for (int A = 0; A < nb; ++A)
+          for (int C = 0; C < nb; ++C) {
+            if (size(A) == 0 || size(C) == 0) continue;
+            const int x = b.spmem[b.spstart[A]], y = b.spmem[b.spstart[C]];
+            if (std::abs(b.tz[x] - b.tz[y]) / 2 != T || (b.ll[x] + b.ll[y]) % 2 != P) continue;
+            if (b.rmap[((size_t)x * N + y) * b.nJ + h] < 0) continue;
+            rowbase[((size_t)h * nb + A) * nb + C] = at;
+            for (int u = b.spstart[A]; u < b.spstart[A + 1]; ++u)
+              for (int w = b.spstart[C]; w < b.spstart[C + 1]; ++w) {
+                if (at >= b.rlen[q] || b.rmap[((size_t)b.spmem[u] * N + b.spmem[w]) * b.nJ + h] < 0) return;
+                B->phb_rows_h[(size_t)b.ccrowoff[q] + at++] = b.spmem[u] | (b.spmem[w] << 16);
+              }
+          }
+        if (at != b.rlen[q]) return;
+      }
+  // quadruples: pairs of blocks A <= B, C <= D of one parity and Tz, {A, B}
+  // up to {C, D}; one {C, D} side by side (neighbours share columns)
+  for (int Pr = 0; Pr <= 1; ++Pr)
+    for (int T = -1; T <= 1; ++T) {
+      std::vector<std::pair<int, int>> sets;
+      for (int A = 0; A < nb; ++A)
+        for (int C = A; C < nb; ++C) {
+          if (size(A) == 0 || size(C) == 0) continue;
+          const int x = b.spmem[b.spstart[A]], y = b.spmem[b.spstart[C]];
+          if ((b.ll[x] + b.ll[y]) % 2 == Pr && (b.tz[x] + b.tz[y]) / 2 == T) sets.push_back({A, C});
+        }
+      for (size_t s2 = 0; s2 < sets.size(); ++s2)
+        for (size_t s1 = 0; s1 <= s2; ++s1) {
+          const int blk[4] = {sets[s1].first, sets[s1].second, sets[s2].first, sets[s2].second};
+          int j[4], l[4], t[4], n[4];
+          for (int x = 0; x < 4; ++x) {
+            const int o = b.spmem[b.spstart[blk[x]]];
+            j[x] = b.jj[o]; l[x] = b.ll[o]; t[x] = b.tz[o];
+            n[x] = size(blk[x]);
+          }
+          PhbQuad Q{};
+          Q.lo = std::max(std::abs(j[0] - j[1]), std::abs(j[2] - j[3]));
+          const int hi = std::min(j[0] + j[1], j[2] + j[3]);
+          if (hi < Q.lo) continue;
+          // the isospin / parity rules of ph_ranges: such elements receive nothing
+          if (std::abs(t[3] - t[1]) != std::abs(t[0] - t[2]) || (l[3] + l[1]) % 2 != (l[0] + l[2]) % 2) continue;
+          if (std::abs(t[2] - t[1]) != std::abs(t[0] - t[3]) || (l[2] + l[1]) % 2 != (l[0] + l[3]) % 2) continue;
+          Q.nJ = (hi - Q.lo) / 2 + 1;
+          Q.jin = std::max(std::abs(j[1] - j[3]), std::abs(j[0] - j[2]));
+          Q.jout = std::max(std::abs(j[0] - j[3]), std::abs(j[1] - j[2]));
+          Q.nin = std::max(0, (std::min(j[1] + j[3], j[0] + j[2]) - Q.jin) / 2 + 1);
+          Q.nout = std::max(0, (std::min(j[0] + j[3], j[1] + j[2]) - Q.jout) / 2 + 1);
+          const int ns = Q.nin + Q.nout;
+          if (ns == 0) continue;
+          if (ns > kPhbSlots) return;
+          Q.slot0 = (int)B->phbs_h.size();
+          for (int s = 0; s < ns; ++s) {
+            const int z = s < Q.nin ? 2 : 3, w = 5 - z;   // i's row partner and the other ket block
+            const int h = (s < Q.nin ? Q.jin + 2 * s : Q.jout + 2 * (s - Q.nin)) / 2;
+            const int q = h + std::abs(t[0] - t[z]) / 2 * (b.JTM + 1) + 2 * ((l[0] + l[z]) % 2) * (b.JTM + 1);
+            auto rb = [&](int x, int y) { return rowbase[((size_t)h * nb + blk[x]) * nb + blk[y]]; };
+            const PhbSlot S{rb(z, 0), rb(1, w), rb(w, 1), rb(0, z), (unsigned)b.wcoff[q], b.rlen[q]};
+            if (S.R1 < 0 || S.C1 < 0 || S.R2 < 0 || S.C2 < 0) return;
+            B->phbs_h.push_back(S);
+          }
+          Q.same = (blk[0] == blk[1] ? 1 : 0) | (blk[2] == blk[3] ? 2 : 0) | (s1 == s2 ? 4 : 0);
+          Q.m = 2 * (T + 1) + Pr;
+          auto pack = [](const int* v) {
+            return (unsigned)v[0] | ((unsigned)v[1] << 8) | ((unsigned)v[2] << 16) | ((unsigned)v[3] << 24);
+          };
+          const int ob[4] = {b.spstart[blk[0]], b.spstart[blk[1]], b.spstart[blk[2]], b.spstart[blk[3]]};
+          Q.ob = pack(ob); Q.N = pack(n); Q.j = pack(j);
+          // at most half the LDS for the coefficients (J cut), then cut B, D, C
+          // and A until the values fit
+          const int lo = Q.lo, nJ = Q.nJ, cJ = std::min(nJ, kPhbLds / 2 / ns);
+          int c[4] = {n[0], n[1], n[2], n[3]};
+          for (int x : {1, 3, 2, 0}) {
+            const int others = c[0] * c[1] * c[2] * c[3] / c[x], m = (kPhbLds - ns * cJ) / (others * ns);
+            c[x] = std::max(1, std::min(c[x], m));
+          }
+          int o[4], m[4];
+          for (int oJ = 0; oJ < nJ; oJ += cJ) {
+            Q.lo = lo + 2 * oJ;
+            Q.nJ = std::min(cJ, nJ - oJ);
+            for (o[0] = 0; o[0] < n[0]; o[0] += c[0])
+            for (o[1] = 0; o[1] < n[1]; o[1] += c[1])
+              for (o[2] = 0; o[2] < n[2]; o[2] += c[2])
+                for (o[3] = 0; o[3] < n[3]; o[3] += c[3]) {
+                  for (int x = 0; x < 4; ++x) m[x] = std::min(c[x], n[x] - o[x]);
+                  Q.off = pack(o); Q.n = pack(m);
+                  B->phbq_h.push_back(Q);
+                }
+          }
+        }
+    }
+  B->phbp.nquads = (int)B->phbq_h.size();
+  B->phb_ok = B->phbp.nquads >= kPhbMinQuads;
+}
+
 int build_plan(imsrg_basis_s* B) {
   const Basis& b = B->b;
   const std::vector<int> order = channel_order(b);
@@ -737,6 +857,7 @@ int build_plan(imsrg_basis_s* B) {
     }
     if (cur.nq > 0) B->phc_h.push_back(cur);
   }
+  build_phb(B);
   // norm chunks: fhh (w 1), fph (w 2), fpp (w 1), gam blocks (w 1 square, 2 rectangular)
   B->ch_off_h.clear(); B->ch_len_h.clear(); B->ch_w_h.clear();
   auto add_range = [&](i64 off, i64 len, double w) {
@@ -798,6 +919,13 @@ int build_plan(imsrg_basis_s* B) {
     return rc;
   if ((rc = upload(B, B->part_h, &B->partners))) return rc;
   if ((rc = upload(B, B->partT_h, &B->partT))) return rc;
+  if (B->phb_ok) {
+    if ((rc = upload(B, B->phbq_h, (PhbQuad**)&B->phbp.quads)) ||
+        (rc = upload(B, B->phbs_h, (PhbSlot**)&B->phbp.slots)) ||
+        (rc = upload(B, B->phb_rows_h, (int**)&B->phbp.rows)) ||
+        (rc = upload(B, B->phb_mem_h, (int**)&B->phbp.mem)))
+      return rc;
+  }
   if (B->t122_ok) {
     if ((rc = upload(B, B->t122_rent, (int**)&B->t122.rent)) || (rc = upload(B, B->t122_rcnt, (int**)&B->t122.rcnt)) ||
         (rc = upload(B, B->t122_rrec, (int2**)&B->t122.rrec)) || (rc = upload(B, B->t122_cent, (int**)&B->t122.cent)) ||
@@ -977,16 +1105,38 @@ void t_221(const Exec& X, const double* L, int Lh, const double* R, int Rh, doub
 void t_pandya(const Exec& X, const double* op, int herm, double* CC, hipStream_t s) {
   run(X.B, X.B->cc, [&](const CCTask* t, int n) { launch_pandya(X.D, t, n, op, herm, CC, s); });
 }
-void t_ph(const Exec& X, const double* LCC, int Lh, const double* RCC, int Rh, double* RES, int RESh,
-          double* WCC, hipStream_t s, bool mirror = true) {
+// W' = Lh LCC RCC^T - Rh RCC LCC^T (upper tiles)
+void t_wprime(const Exec& X, const double* LCC, int Lh, const double* RCC, int Rh, double* WCC, hipStream_t s) {
   imsrg_basis_s* B = X.B;
   Slots sl{};
   sl.p[0] = LCC; sl.p[1] = RCC; sl.p[2] = WCC;
   sl.st[0] = B->b.cclen; sl.st[1] = B->b.cclen; sl.st[2] = B->b.wclen;
   run_gemm_x(X, B->ph, sl, s, (double)Lh, -(double)(Rh * Lh));
+}
+// the cross-coupled form that t_full takes and makes: rows in block order
+// where 222_ph runs by block quadruples
+bool ph_blocks(const Exec& X) { return X.B->phb_ok && X.B->path == IMSRG_PATH_GROUPED; }
+void t_cc(const Exec& X, const double* op, int herm, double* CC, hipStream_t s) {
+  Exec Y = X;
+  if (ph_blocks(X)) Y.D.ccrows = X.B->phbp.rows;
+  t_pandya(Y, op, herm, CC, s);
+}
+// t_full's inverse Pandya on the grouped path: upper triangles
+void t_ph_upper(const Exec& X, const double* WCC, int Lh, int Rh, double* RES, int RESh, hipStream_t s) {
+  imsrg_basis_s* B = X.B;
+  if (ph_blocks(X))
+    launch_comm222ph_blk(X.D, B->phbp, WCC, Lh, Rh, RES, s);
+  else
+    launch_comm222ph_chunk(X.D, B->phc, (int)B->phc_h.size(), B->fq, B->fql, B->fqi, B->quad, WCC, Lh, Rh, RES,
+                           RESh, s, 0);
+}
+void t_ph(const Exec& X, const double* LCC, int Lh, const double* RCC, int Rh, double* RES, int RESh,
+          double* WCC, hipStream_t s) {
+  imsrg_basis_s* B = X.B;
+  t_wprime(X, LCC, Lh, RCC, Rh, WCC, s);
   if (B->path == IMSRG_PATH_GROUPED)
     launch_comm222ph_chunk(X.D, B->phc, (int)B->phc_h.size(), B->fq, B->fql, B->fqi, B->quad, WCC, Lh, Rh, RES,
-                           RESh, s, mirror ? 1 : 0);
+                           RESh, s, 1);
   else
     run(B, B->seg_tri,
         [&](const SegTask* t, int n) { launch_comm222ph_scatter(X.D, t, n, WCC, Lh, Rh, RES, RESh, s); });
@@ -1008,7 +1158,7 @@ void t_norm(const Exec& X, const double* op, double* dst, hipStream_t s) {
 
 // RES = [L, R]: the term sequence of BCH_EXPAND / MAGNUS_EXPAND
 // (IMSRG_MAGNUS.f90:207-219, 677-683).  LCC must already hold the
-// cross-coupled L; RCC is computed here.
+// cross-coupled L (t_cc); RCC is computed here.
 void t_full(const Exec& X, const double* L, int Lh, const double* R, int Rh, double* RES, int RESh, bool e0,
             double* w1, double* w2, const double* LCC, double* RCC, double* WCC, hipStream_t s) {
   // grouped: 122 and 222_ph write the upper triangles of the square blocks
@@ -1028,11 +1178,8 @@ void t_full(const Exec& X, const double* L, int Lh, const double* R, int Rh, dou
     (void)hipEventRecord(ev[0], s);
     for (hipStream_t x : B->aux) (void)hipStreamWaitEvent(x, ev[0], 0);
     // cross-coupled R and W' = Lh LCC RCC^T - Rh RCC LCC^T
-    t_pandya(X, R, Rh, RCC, sc);
-    Slots sw{};
-    sw.p[0] = LCC; sw.p[1] = RCC; sw.p[2] = WCC;
-    sw.st[0] = B->b.cclen; sw.st[1] = B->b.cclen; sw.st[2] = B->b.wclen;
-    run_gemm_x(X, B->ph, sw, sc, (double)Lh, -(double)(Rh * Lh));
+    t_cc(X, R, Rh, RCC, sc);
+    t_wprime(X, LCC, Lh, RCC, Rh, WCC, sc);
     (void)hipEventRecord(ev[1], sc);
     // the 222_pp_hh GEMM families
     const i64 op = B->b.oplen;
@@ -1068,20 +1215,24 @@ void t_full(const Exec& X, const double* L, int Lh, const double* R, int Rh, dou
     (void)hipStreamWaitEvent(s, ev[4], 0);
     t_221(X, L, Lh, R, Rh, RES, RESh, w1, w2, s);
     (void)hipStreamWaitEvent(s, ev[1], 0);
-    launch_comm222ph_chunk(X.D, B->phc, (int)B->phc_h.size(), B->fq, B->fql, B->fqi, B->quad, WCC, Lh, Rh, RES,
-                           RESh, s, 0);
+    t_ph_upper(X, WCC, Lh, Rh, RES, RESh, s);
     launch_sym_lower(X.D, B->symt.dev, B->symt.n, RES, RESh, s);
     return;
   }
-  t_pandya(X, R, Rh, RCC, s);
+  t_cc(X, R, Rh, RCC, s);
   if (e0) t_e0(X, L, Lh, R, Rh, RES, s);
   t_111(X, L, Lh, R, Rh, RES, s);
   t_121(X, L, Lh, R, Rh, RES, RESh, s);
   t_122(X, L, Lh, R, Rh, RES, RESh, s, mirror);
   t_pphh(X, L, Lh, R, Rh, RES, RESh, w1, w2, s, mirror ? 0 : 2);
   t_221(X, L, Lh, R, Rh, RES, RESh, w1, w2, s);
-  t_ph(X, LCC, Lh, RCC, Rh, RES, RESh, WCC, s, mirror);
-  if (!mirror) launch_sym_lower(X.D, X.B->symt.dev, X.B->symt.n, RES, RESh, s);
+  if (mirror) {
+    t_ph(X, LCC, Lh, RCC, Rh, RES, RESh, WCC, s);
+    return;
+  }
+  t_wprime(X, LCC, Lh, RCC, Rh, WCC, s);
+  t_ph_upper(X, WCC, Lh, Rh, RES, RESh, s);
+  launch_sym_lower(X.D, X.B->symt.dev, X.B->symt.n, RES, RESh, s);
 }
 
 
@@ -1542,7 +1693,7 @@ int bch(imsrg_flow_s* F, double* HS, const double* G, int Gh, const double* H, i
   HIPCHK(hipMemcpyAsync(HS, H, n * sizeof(double), hipMemcpyDeviceToDevice, s));
   HIPCHK(hipMemcpyAsync(F->buf[0], H, n * sizeof(double), hipMemcpyDeviceToDevice, s));
   // G is constant over the expansion: its cross-coupled form once
-  t_pandya(F->X, G, Gh, F->GCC, s);
+  t_cc(F->X, G, Gh, F->GCC, s);
   double coef = 1.0;
   int iw;
   for (iw = 2; iw <= maxit; ++iw) {
@@ -1597,7 +1748,7 @@ int magnus(imsrg_flow_s* F, double* DG, int DGh, const double* G, int Gh, double
     rec->c.assign(1, 1.0);
   }
   if (fullnorm < (double)1e-9f) return 0;
-  t_pandya(F->X, G, Gh, F->GCC, s);
+  t_cc(F->X, G, Gh, F->GCC, s);
   int q = 1, cnt = 0;
   for (int i = 2; i <= 7; ++i) {
     double* AD = F->buf[i % 2];
@@ -1661,7 +1812,7 @@ int gen_w2(imsrg_flow_s* F, const Exec& X, const double* H, double* ETA, hipStre
   launch_fill_b(eta1, n, 0.0, X.D.ninst, X.D.act, s);
   if ((rc = gen(X, H, H, eta1, 1, s))) return rc;
   launch_fill_e0(X.D, eta1, 0.0, s);
-  t_pandya(X, eta1, -1, F->GCC, s);
+  t_cc(X, eta1, -1, F->GCC, s);
   t_full(X, eta1, -1, H, 1, H2, 1, true, F->w1, F->w2, F->GCC, F->ADCC, F->WCC, s);
   if ((rc = gen(X, H, H2, ETA, 1, s))) return rc;
   launch_fill_e0(X.D, ETA, 0.0, s);
@@ -1739,7 +1890,7 @@ int bch_b(imsrg_flow_s* F, double* HS, const double* G, const double* H, double 
   if ((rc = set_mask(F, F->acte, F->hme, he, s))) return rc;
   launch_copy_b(HS, H, n, ni, F->acte, s);
   launch_copy_b(F->buf[0], H, n, ni, F->acte, s);
-  t_pandya(F->Xe, G, -1, F->GCC, s);
+  t_cc(F->Xe, G, -1, F->GCC, s);
   double coef = 1.0;
   int iw;
   for (iw = 2; iw <= maxit; ++iw) {
@@ -1799,7 +1950,7 @@ int magnus_b(imsrg_flow_s* F, double* DG, const double* G, double conv, int* nco
   }
   if (!any) return 0;
   if ((rc = set_mask(F, F->acte, F->hme, he, s))) return rc;
-  t_pandya(F->Xe, G, -1, F->GCC, s);
+  t_cc(F->Xe, G, -1, F->GCC, s);
   for (int i = 2; i <= 7; ++i) {
     bool changed = false;
     any = false;
@@ -1873,7 +2024,7 @@ int bch_record(imsrg_flow_s* F, const double* G, const double* H, int Hh, double
   rec.A.assign(1, H);
   rec.c.assign(1, 1.0);
   if (HS) HIPCHK(hipMemcpyAsync(HS, H, n * sizeof(double), hipMemcpyDeviceToDevice, s));
-  t_pandya(F->X, G, -1, F->GCC, s);
+  t_cc(F->X, G, -1, F->GCC, s);
   double coef = 1.0;
   int iw;
   for (iw = 2; iw <= maxit; ++iw) {
@@ -1939,7 +2090,7 @@ int magnus_record(imsrg_flow_s* F, const double* ETA, double* DG, const double* 
   const double fullnorm = B->hval[1];
   if (ncomm) *ncomm = 0;
   if (fullnorm < (double)1e-9f) return 0;
-  t_pandya(F->X, G, -1, F->GCC, s);
+  t_cc(F->X, G, -1, F->GCC, s);
   int q = 1;
   for (int i = 2; i <= 7; ++i) {
     const double adnorm = advals[i - q - 1];
@@ -2049,7 +2200,7 @@ int w2_vjp(imsrg_flow_s* F, const double* H, const double* ETAb, double* Hb, hip
   if ((rc = ensure_adj(B))) return rc;
   launch_fill(F->vE1, n, 0.0, s);
   if ((rc = gen(F->X, H, H, F->vE1, 1, s))) return rc;
-  t_pandya(F->X, F->vE1, -1, F->GCC, s);
+  t_cc(F->X, F->vE1, -1, F->GCC, s);
   t_full(F->X, F->vE1, -1, H, 1, F->vH2, 1, true, F->w1, F->w2, F->GCC, F->ADCC, F->WCC, s);
   launch_axpy(n, ETAb, 1.5, ETAb, 0.0, F->vE1b, s);
   launch_axpy(n, ETAb, 0.5, ETAb, 0.0, F->vE2b, s);
@@ -3009,7 +3160,7 @@ int imsrg_dhds(imsrg_flow F, const double* HS, double* DH, imsrg_stream stream) 
   double* eta = F->tOp;
   launch_fill(eta, F->B->b.oplen, 0.0, s);   // duplicate_sq_op(HS, ETA): a zero operator
   if ((rc = generator(F, F->X, HS, eta, s))) return rc;
-  t_pandya(F->X, eta, -1, F->GCC, s);
+  t_cc(F->X, eta, -1, F->GCC, s);
   t_full(F->X, eta, -1, HS, 1, DH, 1, true, F->w1, F->w2, F->GCC, F->ADCC, F->WCC, s);
   HIPCHK(hipGetLastError());
   return 0;
@@ -3131,7 +3282,7 @@ int imsrg_batch_commutator(imsrg_flow F, const double* L, int Lh, const double* 
   int rc;
   F->hf.assign(F->ninst, 1);
   if ((rc = set_mask(F, F->actf, F->hmf, F->hf, s))) return rc;
-  t_pandya(F->X, L, Lh, F->GCC, s);
+  t_cc(F->X, L, Lh, F->GCC, s);
   t_full(F->X, L, Lh, R, Rh, RES, -Lh * Rh, true, F->w1, F->w2, F->GCC, F->ADCC, F->WCC, s);
   HIPCHK(hipGetLastError());
   return 0;
@@ -3376,14 +3527,13 @@ int imsrg_profile_kernel(imsrg_basis B, int which, const double* L, int Lh, cons
       }
       case IMSRG_K_PH_SCATTER:   // as the grouped commutator runs it: upper triangles only
         if (B->path == IMSRG_PATH_GROUPED)
-          launch_comm222ph_chunk(B->D, B->phc, (int)B->phc_h.size(), B->fq, B->fql, B->fqi, B->quad, WCC, Lh, Rh,
-                                 RES, RESh, s, 0);
+          t_ph_upper(basis_exec(B), WCC, Lh, Rh, RES, RESh, s);
         else
           run(B, B->seg_tri,
               [&](const SegTask* t, int n) { launch_comm222ph_scatter(B->D, t, n, WCC, Lh, Rh, RES, RESh, s); });
         break;
       case IMSRG_K_122: t_122(basis_exec(B), L, Lh, R, Rh, RES, RESh, s, B->path != IMSRG_PATH_GROUPED); break;
-      case IMSRG_K_PANDYA: t_pandya(basis_exec(B), R, Rh, RCC, s); break;
+      case IMSRG_K_PANDYA: t_cc(basis_exec(B), R, Rh, RCC, s); break;
       case IMSRG_K_COPY:   // first half of WCC into its second half: wclen/2 doubles each way
         launch_copy(WCC + B->b.wclen / 2, WCC, B->b.wclen / 2, s);
         break;
@@ -3393,13 +3543,13 @@ int imsrg_profile_kernel(imsrg_basis B, int which, const double* L, int Lh, cons
         t_221(basis_exec(B), L, Lh, R, Rh, RES, RESh, w1, w2, s);
         break;
       case IMSRG_K_COMMUTATOR:
-        t_pandya(basis_exec(B), L, Lh, LCC, s);
+        t_cc(basis_exec(B), L, Lh, LCC, s);
         t_full(basis_exec(B), L, Lh, R, Rh, RES, RESh, true, w1, w2, LCC, RCC, WCC, s);
         break;
     }
   };
   // inputs of every class once (w1/w2, LCC/RCC, WCC), then the timed loop
-  t_pandya(basis_exec(B), L, Lh, LCC, s);
+  t_cc(basis_exec(B), L, Lh, LCC, s);
   t_full(basis_exec(B), L, Lh, R, Rh, RES, RESh, true, w1, w2, LCC, RCC, WCC, s);
   body(which);
   hipEvent_t e0, e1;

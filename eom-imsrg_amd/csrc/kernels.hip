@@ -655,6 +655,167 @@ void launch_comm222ph_chunk(const DevBasis& B, const PhChunk* ch, int nch, const
                      RES, RESh, mirror);
 }
 
+// ------------------------------------------------ 222_ph by block quadruples
+// One wave (workgroup) per quadruple of blocks, or a part of it that fits its
+// LDS; upper triangles of RES only.  The two W' sub-tiles of every
+// (recoupling, J') slot are read along their own contiguous directions and
+// meet in LDS (two additions onto zero: any order gives the same sum); then
+// every output (J, i, j, k, l) sums its quadruple's values against the 6j
+// coefficients of (J, slot).
+// The chunk kernel above gathers single elements of W' (64 lanes, up to 64
+// lines: the address path was busy 90 % of its time, 1.09 GB a launch at eMax 8
+// for 0.41 GB of data); here the lanes run along rows of n_A n_C elements and
+// neighbouring waves share what is left of a line (0.40 GB).  Bound now by
+// vector instructions (index arithmetic: 62 % of the time at eight waves a
+// SIMD).  eMax 7 / 8 / 10: 69 / 182 / 1199 -> 46 / 93 / 642 us.  Tried: one
+// workgroup per 3072 values of several quadruples, searched per lane (194 us at
+// eMax 8, 3200 vector instructions a wave); a wave per quadruple in workgroups
+// of four with 1024 values each (151 us: half the occupancy).
+__device__ __forceinline__ float frcp(int n) { return __builtin_amdgcn_rcpf((float)n); }
+__device__ __forceinline__ int fdiv(int x, float r) { return (int)(((float)x + 0.5f) * r); }   // x / n, r = frcp(n), x < 2^20
+__device__ __forceinline__ void wave_lds_sync() {   // LDS of one wave is in order: hold the compiler only
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// A W' sub-tile with the digits of its contiguous direction (f1 slow, f0
+// fast, stride lf) and of the other one (s1, s0, ls): sizes, value-index
+// strides, offsets of the members taken, the sign of its elements.  A tile of
+// a row block before its column block is stored as it is (rows contiguous),
+// else transposed with the factor -Lh Rh; of a block with itself the lower
+// elements are read transposed.  All of it is wave-uniform.
+struct PhbTile { int nf0, nf1, ns0, lf, ls, of, os, ef0, ef1, es0, es1; double sg; };
+__device__ __forceinline__ PhbTile phb_tile(bool dir, int nr0, int nr1, int nc0, int nc1, int lr, int lc, int orow, int ocol,
+                                            int er0, int er1, int ec0, int ec1, double mpm) {
+  if (dir) return PhbTile{nr0, nr1, nc0, lr, lc, orow, ocol, er0, er1, ec0, ec1, 1.0};
+  return PhbTile{nc0, nc1, nr0, lc, lr, ocol, orow, ec0, ec1, er0, er1, mpm};
+}
+// element e: its value index and its value; F, S the slot's first position in the two directions
+__device__ __forceinline__ double phb_read(const PhbTile& T, float r0, float r1, float r2, int F, int S, unsigned wo,
+                                           unsigned r, int e, const double* WCC, double mpm, int& ev) {
+  const int q0 = fdiv(e, r0), f0 = e - q0 * T.nf0;
+  const int q1 = fdiv(q0, r1), f1 = q0 - q1 * T.nf1;
+  const int s1 = fdiv(q1, r2), s0 = q1 - s1 * T.ns0;
+  ev = __mul24(f0, T.ef0) + __mul24(f1, T.ef1) + __mul24(s0, T.es0) + __mul24(s1, T.es1);
+  const int x = F + __mul24(f1, T.lf) + f0, y = S + __mul24(s1, T.ls) + s0;
+  const double w = WCC[wo + (unsigned)min(x, y) + __umul24((unsigned)max(x, y), r)];
+  return (x <= y ? T.sg : mpm) * w;
+}
+// the slots [s0, s0 + n) of one recoupling: tiles T1, T2 added into v
+__device__ __forceinline__ void phb_slots(const PhbTile& T1, const PhbTile& T2, bool d1, bool d2, const PhbSlot* ss, int s0,
+                                          int n, int n4, const double* WCC, double mpm, int ph, double* v) {
+  const float r4 = frcp(n4), a0 = frcp(T1.nf0), a1 = frcp(T1.nf1), a2 = frcp(T1.ns0);
+  const float b0 = frcp(T2.nf0), b1 = frcp(T2.nf1), b2 = frcp(T2.ns0);
+#pragma unroll 2
+  for (int t = threadIdx.x; t < n * n4; t += 64) {
+    const int q = fdiv(t, r4), e = t - q * n4, s = s0 + q;
+    const PhbSlot S = ss[s];
+    int v1, v2;
+    const double w1 = phb_read(T1, a0, a1, a2, (d1 ? S.R1 : S.C1) + T1.of, (d1 ? S.C1 : S.R1) + T1.os, S.wo, S.r, e, WCC,
+                               mpm, v1);
+    const double w2 = phb_read(T2, b0, b1, b2, (d2 ? S.R2 : S.C2) + T2.of, (d2 ? S.C2 : S.R2) + T2.os, S.wo, S.r, e, WCC,
+                               mpm, v2);
+    unsafeAtomicAdd(&v[s * n4 + v1], w1);
+    unsafeAtomicAdd(&v[s * n4 + v2], ph * w2);
+  }
+}
+
+__global__ __launch_bounds__(64) void k_comm222ph_blk(DevBasis B, PhbPlan P, const double* WCC, int Lh, int Rh,
+                                                      double* RES) {
+  int inst;
+  if (!batch_inst(B, inst)) return;
+  WCC += (i64)inst * B.wclen;
+  RES += (i64)inst * B.oplen;
+  __shared__ double v[kPhbLds];
+  __shared__ PhbSlot ss[kPhbSlots];
+  __shared__ int mem[4 * kPhbMembers];   // members taken of the four blocks
+  const int lane = threadIdx.x;
+  const PhbQuad Q = P.quads[xcd_contig(blockIdx.x, gridDim.x)];   // neighbouring quadruples share lines of W' and RES
+  const double mpm = -(double)(Lh * Rh);
+  const int nA = Q.n & 255, nB = (Q.n >> 8) & 255, nC = (Q.n >> 16) & 255, nD = (Q.n >> 24) & 255;
+  const int NA = Q.N & 255, NB = (Q.N >> 8) & 255, NC = (Q.N >> 16) & 255, ND = (Q.N >> 24) & 255;
+  const int oA = Q.off & 255, oB = (Q.off >> 8) & 255, oC = (Q.off >> 16) & 255, oD = (Q.off >> 24) & 255;
+  const int ji = Q.j & 255, jj = (Q.j >> 8) & 255, jk = (Q.j >> 16) & 255, jl = (Q.j >> 24) & 255;
+  const int nin = Q.nin, ns = nin + Q.nout, n4 = nA * nB * nC * nD, nv = n4 * ns;
+  const float r4 = frcp(n4);
+  if (lane < ns) ss[lane] = P.slots[Q.slot0 + lane];
+  {
+    const int x = 8 * (lane >> 4), y = lane & 15;   // block, member
+    if (y < (int)((Q.n >> x) & 255)) mem[lane] = P.mem[((Q.ob >> x) & 255) + ((Q.off >> x) & 255) + y];
+  }
+  for (int t = lane; t < nv; t += 64) v[t] = 0.0;
+  wave_lds_sync();
+  const int ph = m1pow((ji + jj + jk + jl) / 2);
+  // value index of (i, j, k, l) at one slot: i + nA (k + nC (l + nD j));
+  // in:  W'((k,i),(j,l)) and W'((l,j),(i,k));  out: W'((l,i),(j,k)) and W'((k,j),(i,l)).
+  // Rows are ordered by blocks at every J', so one slot tells the order of all.
+  const int eC = nA, eD = nA * nC, eB = nA * nC * nD;
+  const float rA = frcp(nA), rC = frcp(nC), rD = frcp(nD);
+  if (nin > 0) {
+    const bool d1 = __builtin_amdgcn_readfirstlane(ss[0].R1 <= ss[0].C1), d2 = __builtin_amdgcn_readfirstlane(ss[0].R2 <= ss[0].C2);
+    const PhbTile T1 = phb_tile(d1, nA, nC, nD, nB, NA, ND, oC * NA + oA, oB * ND + oD, 1, eC, eD, eB, mpm);
+    const PhbTile T2 = phb_tile(d2, nB, nD, nC, nA, NB, NC, oD * NB + oB, oA * NC + oC, eB, eD, eC, 1, mpm);
+    phb_slots(T1, T2, d1, d2, ss, 0, nin, n4, WCC, mpm, ph, v);
+  }
+  if (Q.nout > 0) {
+    const bool d1 = __builtin_amdgcn_readfirstlane(ss[nin].R1 <= ss[nin].C1), d2 = __builtin_amdgcn_readfirstlane(ss[nin].R2 <= ss[nin].C2);
+    const PhbTile T1 = phb_tile(d1, nA, nD, nC, nB, NA, NC, oD * NA + oA, oB * NC + oC, 1, eD, eC, eB, mpm);
+    const PhbTile T2 = phb_tile(d2, nB, nC, nD, nA, NB, ND, oC * NB + oB, oA * ND + oD, eB, eC, eD, 1, mpm);
+    phb_slots(T1, T2, d1, d2, ss, nin, Q.nout, n4, WCC, mpm, ph, v);
+  }
+  // 6j coefficients of (J, slot) behind the values
+  double* cof = v + nv;
+  const float rs = frcp(ns);
+  for (int x = lane; x < ns * Q.nJ; x += 64) {
+    const int jx = fdiv(x, rs), s = x - jx * ns, J = Q.lo + 2 * jx;
+    cof[x] = s < nin ? -(double)m1pow((jl + jk + J) / 2) * sixj_tri(B, ji, jj, J, jl, jk, Q.jin + 2 * s)
+                     : sixj_tri(B, ji, jj, J, jk, jl, Q.jout + 2 * (s - nin));
+  }
+  wave_lds_sync();
+  for (int t = lane; t < n4 * Q.nJ; t += 64) {
+    const int jx = fdiv(t, r4), e = t - jx * n4;
+    const int J = Q.lo + 2 * jx;
+    const int x1 = fdiv(e, rA), li = e - x1 * nA;
+    const int x2 = fdiv(x1, rC), lk = x1 - x2 * nC;
+    const int lj = fdiv(x2, rD), ll = x2 - lj * nD;
+    int i = mem[li], j = mem[kPhbMembers + lj], k = mem[2 * kPhbMembers + lk], l = mem[3 * kPhbMembers + ll];
+    const int cp = (i >> 8) + (j >> 8), cq = (k >> 8) + (l >> 8);
+    i &= 255; j &= 255; k &= 255; l &= 255;
+    // pairs of one block are taken in orbit order once, and of {A, B} ==
+    // {C, D} the upper triangle
+    if (((Q.same & 1) && i > j) || ((Q.same & 2) && k > l)) continue;
+    const int ip = B.xmap[(i * B.N + j) * B.nJ + (J >> 1)];
+    const int iq = B.xmap[(k * B.N + l) * B.nJ + (J >> 1)];
+    const bool up = cp < cq || (cp == cq && ip <= iq);   // stored as (ij, kl)
+    if ((Q.same & 4) && !up) continue;
+    const double* cf = cof + jx * ns;
+    const double* vp = v + e;
+    double sm = 0.0;
+    for (int s = 0; s < ns; ++s) sm = fma(cf[s], vp[s * n4], sm);
+    if (i == j) sm *= IMSRG_INV_SQRT2_REF;
+    if (k == l) sm *= IMSRG_INV_SQRT2_REF;
+    // <ij| = -(-1)^((ji + jj - J) / 2) <ji|, and for kl; the lower element by
+    // RES(kl, ij) = -Lh Rh RES(ij, kl)
+    int neg = 0;
+    if (i > j) neg ^= 1 + (ji + jj - J) / 2;
+    if (k > l) neg ^= 1 + (jk + jl - J) / 2;
+    if (neg & 1) sm = -sm;
+    if (!up) sm *= mpm;
+    const int qc = 3 * J + Q.m;
+    const int clo = up ? cp : cq, chi = up ? cq : cp;
+    const int row = up ? ip : iq, col = up ? iq : ip;
+    double* X = RES + B.goff[qc * 6 + blk_of(clo, chi)] + row + (i64)col * B.dims[qc * 3 + clo];
+    *X = *X + sm;
+  }
+}
+
+void launch_comm222ph_blk(const DevBasis& B, const PhbPlan& P, const double* W, int Lh, int Rh, double* RES,
+                          hipStream_t s) {
+  if (P.nquads <= 0) return;
+  hipLaunchKernelGGL(k_comm222ph_blk, dim3(P.nquads, B.ninst), dim3(64), 0, s, B, P, W, Lh, Rh, RES);
+}
+
 // lower triangle of every square block (pppp, phph, hhhh) from its upper
 // triangle: X(y, x) = herm X(x, y) for x < y, by 64 x 64 tile pairs (tile
 // rows ti <= tile columns tj; task.pad = block g) through LDS, coalesced

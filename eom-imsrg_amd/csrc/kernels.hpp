@@ -107,6 +107,35 @@ constexpr int kPhChunkLanes = 1024;
 constexpr int kPhMaxCC = 256;   // cross-coupled blocks whose offsets the chunk kernel keeps in LDS
 struct PhChunk { int q0, nq, item0, nitems, nlanes, pad0, pad1, pad2; };
 
+// 222_ph of the fused commutator by quadruples of (l, j, tz) blocks
+// (k_comm222ph_blk).  The cross-coupled rows of that path are ordered by
+// (block of a, block of b, a, b), so the W' elements that the quadruples (i in
+// block A, j in B, k in C, l in D) read at one J' are four dense sub-tiles, and
+// all of them share their 6j symbols.  One byte per block, A lowest: ob
+// (members' start), N (its members), off and n (the members taken: a
+// quadruple is cut until its values fit the LDS of a wave), j (2j).  nin,
+// nout: J' terms of the two recouplings (slots), from jin / jout; J from lo,
+// nJ values; m: channel part 2 (Tz + 1) + P; same: bit 0 A == B, 1 C == D, 2
+// both pairs equal.
+constexpr int kPhbLds = 512;     // doubles of LDS per quadruple: values and 6j coefficients
+constexpr int kPhbSlots = 48;
+constexpr int kPhbMembers = 16;  // most orbits of a block
+// From about one quadruple a wave slot on: eMax 4 (2491) 13.6 against 9.6 us by
+// chunks, eMax 5 (5349) 13.1 against 13.0, eMax 6 (10276) 26 against 25.7 (and
+// 64 instances of it 3 % faster as a whole), eMax 7 46 against 69, eMax 8 93
+// against 182, eMax 10 642 against 1199 us.
+constexpr int kPhbMinQuads = 4096;
+struct PhbQuad { unsigned ob, N, off, n, j; int same, m, slot0, nin, nout, jin, jout, lo, nJ, pad0, pad1; };
+// a slot's W' block (offset, rows) and the first row / column of its two sub-tiles
+struct PhbSlot { int R1, C1, R2, C2; unsigned wo; int r; };
+struct PhbPlan {
+  const PhbQuad* quads;
+  const PhbSlot* slots;
+  const int* rows;      // the row pairs in block order, packed as ccrows
+  const int* mem;       // block members (the order of spmem), bit 8: hole
+  int nquads;
+};
+
 // One contiguous run of the vectorize stream (basic_IMSRG.f90:3929-3981):
 // len operator elements from op_off map to vector positions vec_off...; for
 // a column of a square block (mirror = its dimension n) repackage also
@@ -157,6 +186,9 @@ void launch_sym_lower(const DevBasis& B, const PairTask* t, int nt, double* RES,
 void launch_comm222ph_chunk(const DevBasis& B, const PhChunk* ch, int nch, const int* fq, const int* fql,
                             const int* fqi, const QuadItem* items, const double* W, int Lh, int Rh, double* RES,
                             int RESh, hipStream_t s, int mirror);
+// 222_ph by block quadruples: upper triangles of RES, W' rows in block order
+void launch_comm222ph_blk(const DevBasis& B, const PhbPlan& P, const double* W, int Lh, int Rh, double* RES,
+                          hipStream_t s);
 // dir 0: vec <- op (vectorize); dir 1: op <- vec (repackage, herm fill)
 void launch_vectorize(const VecTask* t, int nt, double* op, double* vec, int dir, int herm, hipStream_t s);
 // transform_2b_to_HF: gam blocks <-> per-channel square matrices (hh, ph, pp)

@@ -2,10 +2,9 @@
 whose (l, j, tz) blocks select each variant of the kernel (up to 4, 5, 6 and
 7 orbits a block), with partly filled channels and slabs, and on one basis
 with a block too large for a tile and one too small to fill the chip (the
-list kernel).  All four hermiticity
-pairs; RES starts from an unsymmetric prior (the term assigns).  The fused
-commutator (a batch of two operators) covers the form that stores upper
-triangles only."""
+list kernel).  All four hermiticity pairs; RES starts from an unsymmetric
+prior (the term assigns).  The form that stores upper triangles only runs in
+the fused commutator (test_gpu_ph_blocks)."""
 import numpy as np
 import pytest
 import torch
@@ -54,18 +53,3 @@ def test_122_vs_oracle(gpu, emax, lmax, nucleus):
             assert_rel(got[two], ref[two], what=f"122 path {path}")
             assert np.array_equal(got[: two.start], ref[: two.start])
         b.set_path(0)
-
-
-@pytest.mark.parametrize("emax,lmax,nucleus", [(6, 6, "O22"), (8, 4, "C14")])
-def test_commutator_vs_oracle(gpu, emax, lmax, nucleus):
-    from eom_imsrg import Batch
-    b, o = _basis(emax, lmax, nucleus)
-    for hL, hR in HERMS:
-        print(f"[122 tiles, commutator] eMax {emax} lMax {lmax} {nucleus} herm ({hL},{hR})", flush=True)
-        Ls, Rs = [_op(b, hL, s) for s in (5, 6)], [_op(b, hR, s) for s in (7, 8)]
-        bt = Batch(b, 2, graphs=False)
-        RES = bt.zeros()
-        bt.commutator(torch.from_numpy(np.stack(Ls)).cuda(), hL, torch.from_numpy(np.stack(Rs)).cuda(), hR, RES)
-        torch.cuda.synchronize()
-        for k in range(2):
-            assert_rel(RES[k].cpu().numpy(), o.commutator(Ls[k], hL, Rs[k], hR, -hL * hR), what=f"instance {k}")
