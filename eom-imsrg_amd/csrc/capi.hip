@@ -90,12 +90,9 @@ struct imsrg_basis_s {
   Basis b;
   int path = IMSRG_PATH_GROUPED;
   bool dev_ready = false;
-  // GEMM tile shapes for pp1, k2, k3, ph (64x64 until tuned) and the reverse-mode
-  // 222_pp_hh rounds (32x32 through LDS), W' transpose (register-direct 128x64)
-  // and fused pp products (64x32 through LDS, XCD packing): the fastest
-  // commutator transpose at eMax 8 (1.54 ms against 1.62 ms with 64x32, 64x32
-  // and register-direct 128x64)
-  int tile_req[7] = {0, 0, 0, 0, 5, 6, 11};
+  // GEMM tile shapes for pp1, k2, k3, ph and the reverse-mode 222_pp_hh rounds,
+  // W' transpose and fused pp products (default_tiles until the caller sets them)
+  int tile_req[7] = {0, 0, 0, 0, 0, 0, 0};
   int plan_ver = 0;                 // bumped whenever a task list is rebuilt (captured graphs go stale)
   DevBasis D{};
   std::vector<void*> allocs;
@@ -268,6 +265,35 @@ void build_seg(const Basis& b, TaskList<SegTask>& tl, SegMode mode, const std::v
 }
 
 int tiles(int n) { return (n + 63) / 64; }
+
+// Tile shapes of a basis nobody has tuned, from the number of 64 x 64 output
+// tiles of each family.  A launch of few tiles leaves CUs idle and each tile is
+// one long chain of K steps, so small families take 32 x 32 (shape 5); with
+// thousands of tiles the register-direct shapes' higher rate wins.  Measured
+// (us, every family alone, 64x64 / chosen): PPPP eMax 4 9.5 / 6.0, 5 14.9 / 8.7,
+// 6 30 / 17 (307 tiles), 7 60 / 46 (735), 8 162 / 135 (1835), 9 478 / 416; pp x
+// (ph|hh) with its epilogue eMax 5 35 / 26, 7 54 / 43, 9 173 / 151; W' eMax 5 10.3 /
+// 8.3 (294), 7 46 / 43 (2144), 8 105 / 97 (5214), 10 603 / 549 (25410).  Reverse
+// mode, whole commutator transpose: eMax 5 208 -> 185, 6 339 -> 306, 7 723 -> 687,
+// 8 unchanged.
+void default_tiles(imsrg_basis_s* B) {
+  const Basis& b = B->b;
+  i64 pppp = 0, ppx = 0, ph = 0;
+  for (int q = 0; q < b.nblocks; ++q) {
+    const int np = b.dims[q * 3], nx = b.dims[q * 3 + 1] + b.dims[q * 3 + 2];
+    pppp += (i64)tiles(np) * tiles(np);
+    ppx += (i64)tiles(np) * tiles(nx) * ((np + 127) / 128);
+  }
+  for (int q = 0; q < b.ncc; ++q) ph += (i64)tiles(b.rlen[q]) * (tiles(b.rlen[q]) + 1) / 2;
+  const int X = IMSRG_TILE_XCD;
+  B->tile_req[0] = pppp < 512 ? 5 | X : (pppp < 1200 ? 7 | X : 6);
+  B->tile_req[1] = ppx < 700 ? 5 | X : 3 | X;
+  B->tile_req[2] = 5 | X;
+  B->tile_req[3] = ph < 1500 ? 5 | X : (ph < 16000 ? 7 | X : 6 | X);
+  B->tile_req[4] = 5 | X;
+  B->tile_req[5] = ph < 1500 ? 5 | X : (ph < 4000 ? 7 | X : 6);
+  B->tile_req[6] = 3 | X;
+}
 
 // (re)build the tile tasks of a GEMM family for tile shape `tile`.  Groups
 // (channels / cross-coupled blocks) are packed onto the XCDs by cost
@@ -680,8 +706,13 @@ int build_plan(imsrg_basis_s* B) {
     B->k3.group_end.push_back((int)B->k3.probs_h.size());
   }
   B->pairs.n = (int)B->pairs.host.size();
-  B->pp1.tile = B->tile_req[0] & 7; B->k2.tile = B->tile_req[1] & 7; B->k3.tile = B->tile_req[2] & 7;
-  B->ph.tile = B->tile_req[3] & 7;
+  {
+    GemmFamily* f[4] = {&B->pp1, &B->k2, &B->k3, &B->ph};
+    for (int x = 0; x < 4; ++x) {
+      f[x]->tile = B->tile_req[x] & 7;
+      f[x]->xcd_aware = (B->tile_req[x] & IMSRG_TILE_XCD) != 0;
+    }
+  }
   // one-body outputs of 121 / 221 (hh p<=q, pp p<=q, ph), same (l, j, tz)
   B->one_h.clear();
   auto same = [&](int x, int y) { return b.jj[x] == b.jj[y] && b.ll[x] == b.ll[y] && b.tz[x] == b.tz[y]; };
@@ -2576,6 +2607,7 @@ int imsrg_basis_create(int norb, const int* n, const int* l, const int* jj2, con
     delete B;
     return fail(IMSRG_EINVAL, e);
   }
+  default_tiles(B);
   *out = B;
   return 0;
 }

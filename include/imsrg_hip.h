@@ -387,7 +387,8 @@ int imsrg_flow_grad(imsrg_flow f, const double* T, double ds, double bch_conv, d
  * 4 = 32x64, 5 = 32x32 (operands staged through LDS), 6 = 128x64, 7 =
  * 64x64 (register-direct: each wave loads its own 64x32 / 32x32 block's
  * operands, no LDS), plus IMSRG_TILE_XCD to pack each channel's tiles onto
- * one XCD (one L2). */
+ * one XCD (one L2).  Until set, a shape is chosen from the sizes of the
+ * basis (few output tiles: 32x32). */
 #define IMSRG_TILE_XCD 8
 #define IMSRG_GEMM_PPPP 0   /* 222_pp_hh L1 R1 */
 #define IMSRG_GEMM_PPX 1    /* 222_pp_hh pp x (ph|hh) */
