@@ -102,6 +102,7 @@ struct imsrg_basis_s {
   TaskList<CCTask> cc;
   TaskList<PairTask> pairs;
   TaskList<PairTask> symt;          // 64 x 64 tile pairs of every square block (pad = g)
+  TaskList<TailTask> tail;          // tail of a nested commutator: every stored element but E0 once
   GemmFamily pp1, k2, k3, ph;       // pppp L1 R1, pp x (ph|hh), (ph|hh)^2, cross-coupled W'
   // Hartree-Fock two-body transform: T = V M, then V = M^T T per channel
   // (built on first use), with the per-channel square matrices V, T, M
@@ -927,6 +928,30 @@ int build_plan(imsrg_basis_s* B) {
     }
   B->symt.n = (int)B->symt.host.size();
   if ((rc = upload(B, B->symt.host, &B->symt.dev))) return rc;
+  {
+    auto& th = B->tail.host;
+    th.clear();
+    auto run = [&](i64 off, i64 len, double w) {
+      for (i64 x = 0; x < len; x += kTailRun) th.push_back(TailTask{off + x, 0, (int)std::min<i64>(kTailRun, len - x), 0, 0, w});
+    };
+    for (int q = 0; q < b.nblocks; ++q)
+      for (int g = 0; g < 6; ++g) {
+        const i64 off = b.goff[q * 6 + g];
+        if (!kSquare[g]) {
+          run(off, b.blocksize(q, g), 2.0);
+          continue;
+        }
+        const int n = b.dims[q * 3 + (g == 0 ? 0 : (g == 3 ? 1 : 2))];
+        const int nt = (n + kTail - 1) / kTail;
+        for (int tj = 0; tj < nt; ++tj)
+          for (int ti = 0; ti <= tj; ++ti) th.push_back(TailTask{off, n, ti, tj, 0, 1.0});
+      }
+    run(b.off_fhh, (i64)b.A * b.A, 1.0);
+    run(b.off_fph, (i64)b.P * b.A, 2.0);
+    run(b.off_fpp, (i64)b.P * b.P, 1.0);
+    B->tail.n = (int)th.size();
+    if ((rc = upload(B, th, &B->tail.dev))) return rc;
+  }
   // particle-hole pairs inside one (l, j, tz) block (121's intermediate sums)
   {
     std::vector<int> php;
@@ -978,7 +1003,8 @@ int build_plan(imsrg_basis_s* B) {
   if ((rc = dalloc(B, std::max<i64>(k2ofs, 1) * sizeof(double), (void**)&B->K2scr))) return rc;
   B->D.spscr = std::max<i64>(pofs, 1);
   B->D.sk2scr = std::max<i64>(k2ofs, 1);
-  B->npart = std::max<int>(std::max<int>((int)B->ch_off_h.size(), B->seg_g3.n), b.nblocks + 1);
+  B->npart = std::max<int>(std::max<int>((int)B->ch_off_h.size(), B->seg_g3.n),
+                           std::max<int>(B->tail.n, b.nblocks + 1));
   if ((rc = dalloc(B, (size_t)B->npart * sizeof(double), (void**)&B->part))) return rc;
   B->D.spart = B->npart;
   B->D.ninst = 1;
@@ -1187,11 +1213,25 @@ void t_norm(const Exec& X, const double* op, double* dst, hipStream_t s) {
   launch_sum_sqrt_b(X.D, X.part, nch, dst, kDStride, 1, s);
 }
 
+// the end of a grouped t_full: lower triangles, and with ap the append and
+// the norm in the same pass
+struct Append { double* op; double c; double* norm; };   // op += c RES, |RES| into norm
+void t_tail(const Exec& X, double* RES, int RESh, const Append* ap, hipStream_t s) {
+  imsrg_basis_s* B = X.B;
+  if (!ap) {
+    launch_sym_lower(X.D, B->symt.dev, B->symt.n, RES, RESh, s);
+    return;
+  }
+  launch_comm_tail(X.D, B->tail.dev, B->tail.n, RES, RESh, ap->op, ap->c, X.part, s);
+  launch_sum_sqrt_b(X.D, X.part, B->tail.n, ap->norm, kDStride, 1, s);
+}
+
 // RES = [L, R]: the term sequence of BCH_EXPAND / MAGNUS_EXPAND
 // (IMSRG_MAGNUS.f90:207-219, 677-683).  LCC must already hold the
 // cross-coupled L (t_cc); RCC is computed here.
 void t_full(const Exec& X, const double* L, int Lh, const double* R, int Rh, double* RES, int RESh, bool e0,
-            double* w1, double* w2, const double* LCC, double* RCC, double* WCC, hipStream_t s) {
+            double* w1, double* w2, const double* LCC, double* RCC, double* WCC, hipStream_t s,
+            const Append* ap = nullptr) {
   // grouped: 122 and 222_ph write the upper triangles of the square blocks
   // and one symmetrising pass fills the lower ones (every term's
   // contribution is herm-symmetric, so the lower triangles need not be
@@ -1247,7 +1287,7 @@ void t_full(const Exec& X, const double* L, int Lh, const double* R, int Rh, dou
     t_221(X, L, Lh, R, Rh, RES, RESh, w1, w2, s);
     (void)hipStreamWaitEvent(s, ev[1], 0);
     t_ph_upper(X, WCC, Lh, Rh, RES, RESh, s);
-    launch_sym_lower(X.D, B->symt.dev, B->symt.n, RES, RESh, s);
+    t_tail(X, RES, RESh, ap, s);
     return;
   }
   t_cc(X, R, Rh, RCC, s);
@@ -1259,11 +1299,12 @@ void t_full(const Exec& X, const double* L, int Lh, const double* R, int Rh, dou
   t_221(X, L, Lh, R, Rh, RES, RESh, w1, w2, s);
   if (mirror) {
     t_ph(X, LCC, Lh, RCC, Rh, RES, RESh, WCC, s);
+    if (ap) t_axpy_norm(X, ap->op, RES, ap->c, ap->norm, s);
     return;
   }
   t_wprime(X, LCC, Lh, RCC, Rh, WCC, s);
   t_ph_upper(X, WCC, Lh, Rh, RES, RESh, s);
-  launch_sym_lower(X.D, X.B->symt.dev, X.B->symt.n, RES, RESh, s);
+  t_tail(X, RES, RESh, ap, s);
 }
 
 
@@ -1734,8 +1775,8 @@ int bch(imsrg_flow_s* F, double* HS, const double* G, int Gh, const double* H, i
     const double c = coef;
     imsrg_flow_s::GraphKey key{0, iw, HS, G, H, Gh, Hh};
     int rc = run_term(F, key, s, [&](hipStream_t cs) {
-      t_full(F->X, G, Gh, AD, Hh, INT2, Hh, true, F->w1, F->w2, F->GCC, F->ADCC, F->WCC, cs);
-      t_axpy_norm(F->X, HS, INT2, c, B->dval, cs);
+      const Append ap{HS, c, B->dval};
+      t_full(F->X, G, Gh, AD, Hh, INT2, Hh, true, F->w1, F->w2, F->GCC, F->ADCC, F->WCC, cs, &ap);
     });
     if (rc) return rc;
     if (rec) {
@@ -1790,8 +1831,8 @@ int magnus(imsrg_flow_s* F, double* DG, int DGh, const double* G, int Gh, double
     const double c = cof[i - 1];
     imsrg_flow_s::GraphKey key{1, i, DG, G, nullptr, Gh, DGh};
     rc = run_term(F, key, s, [&](hipStream_t cs) {
-      t_full(F->X, G, Gh, AD, DGh, INT2, DGh, false, F->w1, F->w2, F->GCC, F->ADCC, F->WCC, cs);
-      t_axpy_norm(F->X, DG, INT2, c, B->dval, cs);
+      const Append ap{DG, c, B->dval};
+      t_full(F->X, G, Gh, AD, DGh, INT2, DGh, false, F->w1, F->w2, F->GCC, F->ADCC, F->WCC, cs, &ap);
     });
     if (rc) return rc;
     ++cnt;
@@ -1931,8 +1972,8 @@ int bch_b(imsrg_flow_s* F, double* HS, const double* G, const double* H, double 
     const double c = coef;
     imsrg_flow_s::GraphKey key{2, iw, HS, G, H, -1, 1};
     rc = run_term(F, key, s, [&](hipStream_t cs) {
-      t_full(F->Xe, G, -1, AD, 1, INT2, 1, true, F->w1, F->w2, F->GCC, F->ADCC, F->WCC, cs);
-      t_axpy_norm(F->Xe, HS, INT2, c, F->Xe.dval, cs);
+      const Append ap{HS, c, F->Xe.dval};
+      t_full(F->Xe, G, -1, AD, 1, INT2, 1, true, F->w1, F->w2, F->GCC, F->ADCC, F->WCC, cs, &ap);
     });
     if (rc) return rc;
     if ((rc = read_inst(F, 1, nullptr, s))) return rc;
@@ -2003,8 +2044,8 @@ int magnus_b(imsrg_flow_s* F, double* DG, const double* G, double conv, int* nco
     const double c = cof[i - 1];
     imsrg_flow_s::GraphKey key{3, i, DG, G, nullptr, -1, -1};
     rc = run_term(F, key, s, [&](hipStream_t cs) {
-      t_full(F->Xe, G, -1, AD, -1, INT2, -1, false, F->w1, F->w2, F->GCC, F->ADCC, F->WCC, cs);
-      t_axpy_norm(F->Xe, DG, INT2, c, F->Xe.dval, cs);
+      const Append ap{DG, c, F->Xe.dval};
+      t_full(F->Xe, G, -1, AD, -1, INT2, -1, false, F->w1, F->w2, F->GCC, F->ADCC, F->WCC, cs, &ap);
     });
     if (rc) return rc;
     if ((rc = read_inst(F, 1, nullptr, s))) return rc;
@@ -2062,9 +2103,9 @@ int bch_record(imsrg_flow_s* F, const double* G, const double* H, int Hh, double
     coef = coef / (iw - 1.0);
     double* nx = nullptr;
     if ((rc = pool_get(F, pidx, &nx))) return rc;
-    t_full(F->X, G, -1, rec.A.back(), Hh, nx, Hh, true, F->w1, F->w2, F->GCC, F->ADCC, F->WCC, s);
-    if (HS) launch_axpy(n, HS, 1.0, nx, coef, HS, s);
-    t_norm(F->X, nx, B->dval, s);
+    const Append ap{HS, coef, B->dval};
+    t_full(F->X, G, -1, rec.A.back(), Hh, nx, Hh, true, F->w1, F->w2, F->GCC, F->ADCC, F->WCC, s, HS ? &ap : nullptr);
+    if (!HS) t_norm(F->X, nx, B->dval, s);
     double nrm = 0.0;
     if ((rc = read_scalar(B, B->dval, &nrm, s))) return rc;
     rec.A.push_back(nx);
@@ -2130,9 +2171,8 @@ int magnus_record(imsrg_flow_s* F, const double* ETA, double* DG, const double* 
     double* nx = nullptr;
     if ((rc = pool_get(F, pidx, &nx))) return rc;
     HIPCHK(hipMemcpyAsync(nx, rec.A.back(), sizeof(double), hipMemcpyDeviceToDevice, s));
-    t_full(F->X, G, -1, rec.A.back(), -1, nx, -1, false, F->w1, F->w2, F->GCC, F->ADCC, F->WCC, s);
-    launch_axpy(n, DG, 1.0, nx, cof[i - 1], DG, s);
-    t_norm(F->X, nx, B->dval, s);
+    const Append ap{DG, cof[i - 1], B->dval};
+    t_full(F->X, G, -1, rec.A.back(), -1, nx, -1, false, F->w1, F->w2, F->GCC, F->ADCC, F->WCC, s, &ap);
     double nrm = 0.0;
     if ((rc = read_scalar(B, B->dval, &nrm, s))) return rc;
     advals[i - 1] = nrm * std::fabs(cof[i - 1]);

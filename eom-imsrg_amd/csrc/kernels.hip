@@ -78,25 +78,24 @@ __device__ __forceinline__ double sum122(double sm, const Partner* part, i64 ps,
   return sm;
 }
 
-__global__ __launch_bounds__(256) void k_comm122p(DevBasis B, const SegTask* tasks, const Partner* part,
-                                                  const Partner* partT, int pstride, const int* rowp,
-                                                  const int* colp, const int* f1off, int nf1,
-                                                  const double* L, int Lh, const double* R, int Rh, double* RES,
-                                                  int RESh, int mirror) {
+__device__ __forceinline__ void d_comm122p(DevBasis B, const SegTask* tasks, const Partner* part,
+                                           const Partner* partT, int pstride, const int* rowp, const int* colp,
+                                           const int* f1off, int nf1, const double* L, int Lh, const double* R,
+                                           int Rh, double* RES, int RESh, int mirror, int bx, int nbx,
+                                           double* s_f) {
   int inst;
   if (!batch_inst(B, inst)) return;
   L += (i64)inst * B.oplen;
   R += (i64)inst * B.oplen;
   RES += (i64)inst * B.oplen;
   // the one-body elements the partner terms read, L then R, staged once
-  extern __shared__ double s_f[];
   for (int k = threadIdx.x; k < nf1; k += blockDim.x) {
     const int o = f1off[k];
     s_f[k] = L[o];
     s_f[nf1 + k] = R[o];
   }
   __syncthreads();
-  const SegTask t = tasks[xcd_contig(blockIdx.x, gridDim.x)];   // neighbouring tiles share partner rows
+  const SegTask t = tasks[xcd_contig(bx, nbx)];   // neighbouring tiles share partner rows
   const i64 e = (i64)t.start + threadIdx.x;
   if (e >= t.cnt) return;
   const int q = t.q, g = t.g;
@@ -133,6 +132,15 @@ __global__ __launch_bounds__(256) void k_comm122p(DevBasis B, const SegTask* tas
   const i64 base = B.goff[q * 6 + g];
   RES[base + IX + (i64)JX * n1] = sm;
   if (sq && mirror) RES[base + JX + (i64)IX * n1] = sm * RESh;
+}
+
+__global__ __launch_bounds__(256) void k_comm122p(DevBasis B, const SegTask* tasks, const Partner* part,
+                                                  const Partner* partT, int pstride, const int* rowp,
+                                                  const int* colp, const int* f1off, int nf1, const double* L,
+                                                  int Lh, const double* R, int Rh, double* RES, int RESh,
+                                                  int mirror) {
+  extern __shared__ double s_f[];
+  d_comm122p(B, tasks, part, partT, pstride, rowp, colp, f1off, nf1, L, Lh, R, Rh, RES, RESh, mirror, blockIdx.x, gridDim.x, s_f);
 }
 
 void launch_comm122p(const DevBasis& B, const SegTask* t, int nt, const Partner* part, const Partner* partT,
@@ -552,25 +560,31 @@ __device__ __forceinline__ int lds_floor(const int* a, int n, int t) {
 // quadruple's terms from LDS with the 6j weights, in the order ph_element
 // adds them (same result bits).  Each W' term is fetched once per
 // quadruple instead of once per (quadruple, J).
-__global__ __launch_bounds__(256) void k_comm222ph_chunk(DevBasis B, const PhChunk* chunks, const int* fq,
-                                                         const int* fql, const int* fqi, const QuadItem* items,
-                                                         const double* WCC, int Lh, int Rh, double* RES, int RESh,
-                                                         int mirror) {
-  int inst;
-  if (!batch_inst(B, inst)) return;
-  WCC += (i64)inst * B.wclen;
-  RES += (i64)inst * B.oplen;
-  __shared__ int s_ijkl[kPhChunkItems], s_loff[kPhChunkItems], s_ioff[kPhChunkItems];
-  __shared__ int s_jin[kPhChunkItems], s_nin[kPhChunkItems], s_jout[kPhChunkItems];
+struct PhChunkLds {
+  int ijkl[kPhChunkItems], loff[kPhChunkItems], ioff[kPhChunkItems];
+  int jin[kPhChunkItems], nin[kPhChunkItems], jout[kPhChunkItems];
   // per quadruple, from the orbit tables once: 2j of i, j, k, l (8 bits
   // each), and the recoupling / output data (phase, Tz and parity of the
   // inside and outside recouplings, the output channel's Tz / parity part,
   // block g and the two (a,a) factors)
-  __shared__ int s_jq[kPhChunkItems], s_meta[kPhChunkItems];
-  __shared__ double s_val[kPhChunkLanes];
-  __shared__ i64 s_wcoff[kPhMaxCC];
-  __shared__ int s_rlen[kPhMaxCC];
-  const PhChunk c = chunks[xcd_contig(blockIdx.x, gridDim.x)];   // neighbouring chunks share W' lines
+  int jq[kPhChunkItems], meta[kPhChunkItems];
+  double val[kPhChunkLanes];
+  i64 wcoff[kPhMaxCC];
+  int rlen[kPhMaxCC];
+};
+__device__ __forceinline__ void d_comm222ph_chunk(const DevBasis& B, const PhChunk* chunks, const int* fq,
+                                                  const int* fql, const int* fqi, const QuadItem* items,
+                                                  const double* WCC, int Lh, int Rh, double* RES, int RESh, int mirror,
+                                                  int bx, int nbx, PhChunkLds& S) {
+  int inst;
+  if (!batch_inst(B, inst)) return;
+  WCC += (i64)inst * B.wclen;
+  RES += (i64)inst * B.oplen;
+  int *s_ijkl = S.ijkl, *s_loff = S.loff, *s_ioff = S.ioff, *s_jin = S.jin, *s_nin = S.nin, *s_jout = S.jout;
+  int *s_jq = S.jq, *s_meta = S.meta, *s_rlen = S.rlen;
+  double* s_val = S.val;
+  i64* s_wcoff = S.wcoff;
+  const PhChunk c = chunks[xcd_contig(bx, nbx)];   // neighbouring chunks share W' lines
   const int tid = threadIdx.x;
   const double mpm = -(double)(Lh * Rh);
   for (int x = tid; x < B.ncc; x += blockDim.x) {   // cross-coupled block offsets and row counts
@@ -645,6 +659,13 @@ __global__ __launch_bounds__(256) void k_comm222ph_chunk(DevBasis B, const PhChu
   const i64 o = IX + (i64)JX * n1;
   X[o] = X[o] + sm * pre * pre2;
   if (is_square(g) && mirror) X[JX + (i64)IX * n1] = X[o] * RESh;
+}
+__global__ __launch_bounds__(256) void k_comm222ph_chunk(DevBasis B, const PhChunk* chunks, const int* fq,
+                                                         const int* fql, const int* fqi, const QuadItem* items,
+                                                         const double* WCC, int Lh, int Rh, double* RES, int RESh,
+                                                         int mirror) {
+  __shared__ PhChunkLds S;
+  d_comm222ph_chunk(B, chunks, fq, fql, fqi, items, WCC, Lh, Rh, RES, RESh, mirror, blockIdx.x, gridDim.x, S);
 }
 
 void launch_comm222ph_chunk(const DevBasis& B, const PhChunk* ch, int nch, const int* fq, const int* fql,
@@ -851,13 +872,13 @@ void launch_sym_lower(const DevBasis& B, const PairTask* t, int nt, double* RES,
 // =========================================================== Pandya forward
 // calculate_cross_coupled, cross_coupled.f90:1190-1300.  One thread per
 // CCX(q1)(r, nb) element; r = ordered pair (a,b), nb = (p,h).
-__global__ __launch_bounds__(256) void k_pandya(DevBasis B, const CCTask* tasks, const double* op, int herm,
-                                                double* CC) {
+__device__ __forceinline__ void d_pandya(DevBasis B, const CCTask* tasks, const double* op, int herm, double* CC,
+                                         int bx, int nbx) {
   int inst;
   if (!batch_inst(B, inst)) return;
   op += (i64)inst * B.oplen;
   CC += (i64)inst * B.cclen;
-  const CCTask t = tasks[xcd_contig(blockIdx.x, gridDim.x)];
+  const CCTask t = tasks[xcd_contig(bx, nbx)];
   const int q1 = t.q1;
   const int r = B.rlen[q1], nc = B.ncol[q1];
   const i64 e = (i64)t.start + threadIdx.x;
@@ -883,6 +904,11 @@ __global__ __launch_bounds__(256) void k_pandya(DevBasis B, const CCTask* tasks,
   CC[B.ccoff[q1] + R + (i64)NB * r] = val;
 }
 
+__global__ __launch_bounds__(256) void k_pandya(DevBasis B, const CCTask* tasks, const double* op, int herm,
+                                                double* CC) {
+  d_pandya(B, tasks, op, herm, CC, blockIdx.x, gridDim.x);
+}
+
 void launch_pandya(const DevBasis& B, const CCTask* t, int nt, const double* op, int herm, double* CC,
                    hipStream_t s) {
   if (nt <= 0) return;
@@ -893,15 +919,15 @@ void launch_pandya(const DevBasis& B, const CCTask* t, int nt, const double* op,
 // commutators.f90:36-80.  One wave per one-body output (assigns); the lanes
 // split the intermediate orbit k and the partial dot products are reduced
 // across the wave.
-__global__ __launch_bounds__(256) void k_comm111(DevBasis B, const double* L, int Lh, const double* R, int Rh,
-                                                 double* RES) {
+__device__ __forceinline__ void d_comm111(DevBasis B, const double* L, int Lh, const double* R, int Rh,
+                                          double* RES, int bx) {
   int inst;
   if (!batch_inst(B, inst)) return;
   L += (i64)inst * B.oplen;
   R += (i64)inst * B.oplen;
   RES += (i64)inst * B.oplen;
   const int A = B.A, P = B.P;
-  const i64 idx = (i64)blockIdx.x * 4 + (threadIdx.x >> 6);   // wave-uniform
+  const i64 idx = (i64)bx * 4 + (threadIdx.x >> 6);   // wave-uniform
   const int lane = threadIdx.x & 63;
   const double *Lhh = L + B.off_fhh, *Lph = L + B.off_fph, *Lpp = L + B.off_fpp;
   const double *Rhh = R + B.off_fhh, *Rph = R + B.off_fph, *Rpp = R + B.off_fpp;
@@ -951,6 +977,11 @@ __global__ __launch_bounds__(256) void k_comm111(DevBasis B, const double* L, in
   }
 }
 
+__global__ __launch_bounds__(256) void k_comm111(DevBasis B, const double* L, int Lh, const double* R, int Rh,
+                                                 double* RES) {
+  d_comm111(B, L, Lh, R, Rh, RES, blockIdx.x);
+}
+
 void launch_comm111(const DevBasis& B, const double* L, int Lh, const double* R, int Rh, double* RES,
                     hipStream_t s) {
   const i64 n = (i64)B.A * B.A + (i64)B.P * B.A + (i64)B.P * B.P;
@@ -985,15 +1016,14 @@ __device__ __forceinline__ void onebody_update(const DevBasis& B, const OneTask&
 // (p, q); its threads take the (particle a, hole i, J) terms, with (a, i)
 // from the list of particle-hole pairs inside one (l, j, tz) block (the
 // only pairs the reference's loop keeps), tree-reduced in LDS.
-__global__ __launch_bounds__(256) void k_comm121(DevBasis B, const OneTask* tasks, const double* L, int Lh,
-                                                 const double* R, int Rh, double* RES, int RESh) {
-  __shared__ double red[256];
+__device__ __forceinline__ void d_comm121(DevBasis B, const OneTask* tasks, const double* L, int Lh,
+                                          const double* R, int Rh, double* RES, int RESh, int bx, double* red) {
   int inst;
   if (!batch_inst(B, inst)) return;
   L += (i64)inst * B.oplen;
   R += (i64)inst * B.oplen;
   RES += (i64)inst * B.oplen;
-  const OneTask t = tasks[blockIdx.x];
+  const OneTask t = tasks[bx];
   const int pk = t.pk, qk = t.qk, jq = B.jj[qk];
   const double* Lph = L + B.off_fph;
   const double* Rph = R + B.off_fph;
@@ -1013,6 +1043,12 @@ __global__ __launch_bounds__(256) void k_comm121(DevBasis B, const OneTask* task
   }
   const double sm = block_sum(v, red);
   if (threadIdx.x == 0) onebody_update(B, t, sm / (B.jj[pk] + 1.0), RES, RESh);
+}
+
+__global__ __launch_bounds__(256) void k_comm121(DevBasis B, const OneTask* tasks, const double* L, int Lh,
+                                                 const double* R, int Rh, double* RES, int RESh) {
+  __shared__ double red[256];
+  d_comm121(B, tasks, L, Lh, R, Rh, RES, RESh, blockIdx.x, red);
 }
 
 void launch_comm121(const DevBasis& B, const OneTask* t, int nt, const double* L, int Lh, const double* R,
@@ -1043,10 +1079,9 @@ __device__ __forceinline__ double w2_elem(const DevBasis& B, const double* w2, c
   return (s * Rh) * p.pre;
 }
 
-__global__ __launch_bounds__(256) void k_comm221(DevBasis B, const OneTask* tasks, const double* L, int Lh,
-                                                 const double* R, int Rh, const double* w1, const double* w2,
-                                                 double* RES, int RESh) {
-  __shared__ double red[256];
+__device__ __forceinline__ void d_comm221(DevBasis B, const OneTask* tasks, const double* L, int Lh,
+                                          const double* R, int Rh, const double* w1, const double* w2,
+                                          double* RES, int RESh, int bx, double* red) {
   int inst;
   if (!batch_inst(B, inst)) return;
   L += (i64)inst * B.oplen;
@@ -1054,7 +1089,7 @@ __global__ __launch_bounds__(256) void k_comm221(DevBasis B, const OneTask* task
   w1 += (i64)inst * B.oplen;
   w2 += (i64)inst * B.oplen;
   RES += (i64)inst * B.oplen;
-  const OneTask t = tasks[blockIdx.x];
+  const OneTask t = tasks[bx];
   const int ik = t.pk, jk = t.qk, ji = B.jj[ik];
   const int pm = Lh * Rh;
   const bool both = (t.kind != 2);
@@ -1086,6 +1121,13 @@ __global__ __launch_bounds__(256) void k_comm221(DevBasis B, const OneTask* task
   if (threadIdx.x == 0) onebody_update(B, t, sm / (ji + 1.0), RES, RESh);
 }
 
+__global__ __launch_bounds__(256) void k_comm221(DevBasis B, const OneTask* tasks, const double* L, int Lh,
+                                                 const double* R, int Rh, const double* w1, const double* w2,
+                                                 double* RES, int RESh) {
+  __shared__ double red[256];
+  d_comm221(B, tasks, L, Lh, R, Rh, w1, w2, RES, RESh, blockIdx.x, red);
+}
+
 void launch_comm221(const DevBasis& B, const OneTask* t, int nt, const double* L, int Lh, const double* R, int Rh,
                     const double* w1, const double* w2, double* RES, int RESh, hipStream_t s) {
   if (nt <= 0) return;
@@ -1108,15 +1150,14 @@ __device__ double block_sum(double v, double* red) {
   return r;
 }
 
-__global__ __launch_bounds__(256) void k_e0_partials(DevBasis B, const double* L, int Lh, const double* R, int Rh,
-                                                     double* part) {
+__device__ __forceinline__ void d_e0_partials(DevBasis B, const double* L, int Lh, const double* R, int Rh,
+                                              double* part, int bx, double* red) {
   int inst;
   if (!batch_inst(B, inst)) return;
   L += (i64)inst * B.oplen;
   R += (i64)inst * B.oplen;
   part += (i64)inst * B.spart;
-  __shared__ double red[256];
-  const int q = blockIdx.x;
+  const int q = bx;
   double v = 0.0;
   if (q < B.nblocks) {
     const int np = B.dims[q * 3], nh = B.dims[q * 3 + 2];
@@ -1137,10 +1178,15 @@ __global__ __launch_bounds__(256) void k_e0_partials(DevBasis B, const double* L
   }
 }
 
-// dst = [use110] part[n] + [use220] 2 * sum(part[0..n-1])   (one workgroup)
-__global__ __launch_bounds__(256) void k_e0_final(const double* part, int n, int use220, int use110, double* dst,
-                                                  int accumulate, i64 spart, i64 sdst, const int* act) {
+__global__ __launch_bounds__(256) void k_e0_partials(DevBasis B, const double* L, int Lh, const double* R,
+                                                     int Rh, double* part) {
   __shared__ double red[256];
+  d_e0_partials(B, L, Lh, R, Rh, part, blockIdx.x, red);
+}
+
+// dst = [use110] part[n] + [use220] 2 * sum(part[0..n-1])   (one workgroup)
+__device__ __forceinline__ void d_e0_final(const double* part, int n, int use220, int use110, double* dst,
+                                           int accumulate, i64 spart, i64 sdst, const int* act, double* red) {
   int inst;
   if (!batch_on(act, inst)) return;
   part += (i64)inst * spart;
@@ -1154,6 +1200,12 @@ __global__ __launch_bounds__(256) void k_e0_final(const double* part, int n, int
     const double e = e110 + e220;
     dst[0] = accumulate ? dst[0] + e : e;
   }
+}
+
+__global__ __launch_bounds__(256) void k_e0_final(const double* part, int n, int use220, int use110, double* dst,
+                                                  int accumulate, i64 spart, i64 sdst, const int* act) {
+  __shared__ double red[256];
+  d_e0_final(part, n, use220, use110, dst, accumulate, spart, sdst, act, red);
 }
 
 void launch_e0_partials(const DevBasis& B, const double* L, int Lh, const double* R, int Rh, double* part,
@@ -1249,18 +1301,18 @@ __global__ __launch_bounds__(256) void k_pppp_sym(DevBasis B, const PairTask* ta
 // + side), its own C tile read straight from memory and only the tile whose
 // transpose it needs staged in LDS (33 KB instead of 66 KB: twice the
 // workgroups per CU).  Same arithmetic as k_pppp_sym.
-__global__ __launch_bounds__(256) void k_pppp_sym1(DevBasis B, const PairTask* tasks, double* RES, const double* w1,
-                                                   int pm, int upper_only) {
+__device__ __forceinline__ void d_pppp_sym1(DevBasis B, const PairTask* tasks, double* RES, const double* w1,
+                                            int pm, int upper_only, int bx, double (*S)[65]) {
   int inst;
   if (!batch_inst(B, inst)) return;
   RES += (i64)inst * B.oplen;
   w1 += (i64)inst * B.oplen;
-  __shared__ double S[64][65];   // S[x][y] = C(A0 + x, B0 + y), the transposed source tile
+  // S[x][y] = C(A0 + x, B0 + y), the transposed source tile
   // upper_only: one workgroup per tile pair for its upper tile (the caller
   // fills the lower triangles afterwards), else two, the second for the
   // lower tile
-  const PairTask t = tasks[upper_only ? blockIdx.x : blockIdx.x >> 1];
-  const int side = upper_only ? 0 : (blockIdx.x & 1);
+  const PairTask t = tasks[upper_only ? bx : bx >> 1];
+  const int side = upper_only ? 0 : (bx & 1);
   if (side == 1 && t.ti == t.tj) return;
   const int q = t.q;
   const int np = B.dims[q * 3];
@@ -1284,6 +1336,12 @@ __global__ __launch_bounds__(256) void k_pppp_sym1(DevBasis B, const PairTask* t
       X1[o] = X1[o] + cxy - cyx * pm;
     }
   }
+}
+
+__global__ __launch_bounds__(256) void k_pppp_sym1(DevBasis B, const PairTask* tasks, double* RES,
+                                                   const double* w1, int pm, int upper_only) {
+  __shared__ double S[64][65];
+  d_pppp_sym1(B, tasks, RES, w1, pm, upper_only, blockIdx.x, S);
 }
 
 void launch_pppp_sym(const DevBasis& B, const PairTask* t, int nt, const double* L, int Lh, const double* R, int Rh,
@@ -1310,11 +1368,10 @@ __device__ __forceinline__ double pval(const double* Pq, int nbh, int ks, int x,
   return v;
 }
 
-__global__ __launch_bounds__(256) void k_pphh_epilogue(DevBasis B, const SegTask* tasks, const double* L, int Lh,
-                                                       const double* R, int Rh, double* RES, double* w1,
-                                                       double* w2, const double* Pscr, const i64* poff,
-                                                       const int* k3ks, const double* K2scr, const i64* k2off,
-                                                       const int* k2ks) {
+__device__ __forceinline__ void d_pphh_epilogue(DevBasis B, const SegTask* tasks, const double* L, int Lh,
+                                                const double* R, int Rh, double* RES, double* w1, double* w2,
+                                                const double* Pscr, const i64* poff, const int* k3ks,
+                                                const double* K2scr, const i64* k2off, const int* k2ks, int bx) {
   int inst;
   if (!batch_inst(B, inst)) return;
   L += (i64)inst * B.oplen;
@@ -1324,7 +1381,7 @@ __global__ __launch_bounds__(256) void k_pphh_epilogue(DevBasis B, const SegTask
   w2 += (i64)inst * B.oplen;
   Pscr += (i64)inst * B.spscr;
   K2scr += (i64)inst * B.sk2scr;
-  const SegTask t = tasks[blockIdx.x];
+  const SegTask t = tasks[bx];
   const i64 e = (i64)t.start + threadIdx.x;
   if (e >= t.cnt) return;
   const int q = t.q;
@@ -1411,6 +1468,14 @@ __global__ __launch_bounds__(256) void k_pphh_epilogue(DevBasis B, const SegTask
   }
 }
 
+__global__ __launch_bounds__(256) void k_pphh_epilogue(DevBasis B, const SegTask* tasks, const double* L, int Lh,
+                                                       const double* R, int Rh, double* RES, double* w1,
+                                                       double* w2, const double* Pscr, const i64* poff,
+                                                       const int* k3ks, const double* K2scr, const i64* k2off,
+                                                       const int* k2ks) {
+  d_pphh_epilogue(B, tasks, L, Lh, R, Rh, RES, w1, w2, Pscr, poff, k3ks, K2scr, k2off, k2ks, blockIdx.x);
+}
+
 void launch_pphh_epilogue(const DevBasis& B, const SegTask* t, int nt, const double* L, int Lh, const double* R,
                           int Rh, double* RES, double* w1, double* w2, const double* Pscr, const i64* poff,
                           const int* k3ks, const double* K2scr, const i64* k2off, const int* k2ks, hipStream_t s) {
@@ -1464,6 +1529,80 @@ __global__ __launch_bounds__(256) void k_norm_partials(const double* op, const i
   const double s = block_sum(v, red);
   if (threadIdx.x == 0) part[c] = s * cw[c];
 }
+// The tail of one nested commutator in one pass over its result T: lower
+// triangles of the square blocks T(y, x) = herm T(x, y), X += c * T (E0 by
+// task 0's first thread) and the norm partials of T (append_operator +
+// mat_frob_norm, IMSRG_MAGNUS.f90:227-229).  Memory bound, and at small sizes
+// the latency of one load -> LDS -> store chain: a task is a kTail x kTail
+// tile pair of a square block (upper tile through LDS, every load issued
+// before the barrier) or a run of at most kTailRun elements of T outside
+// them.  Against symmetrising and then appending in a second pass: decoupling
+// eMax 4 23.3 -> 21.6 ms, BCH eMax 6 (22O) 3.71 -> 3.42 ms, eMax 10 70.9 ->
+// 70.1 ms; 32-wide tiles keep all loads of a thread in registers (51 VGPRs,
+// 8 waves a SIMD).
+__global__ __launch_bounds__(256) void k_comm_tail(DevBasis B, const TailTask* tasks, double* T, int herm, double* X,
+                                                   double c, double* part) {
+  __shared__ double S[kTail][kTail + 1];
+  __shared__ double red[256];
+  int inst;
+  if (!batch_inst(B, inst)) return;
+  X += (i64)inst * B.oplen;
+  T += (i64)inst * B.oplen;
+  part += (i64)inst * B.spart;
+  const TailTask t = tasks[blockIdx.x];
+  if (blockIdx.x == 0 && threadIdx.x == 0) X[0] = X[0] * 1.0 + T[0] * c;
+  double v = 0.0;
+  const int n = t.n;
+  if (n > 0) {
+    constexpr int C = kTail * kTail / 256;
+    double* Tb = T + t.off;
+    double* Xb = X + t.off;
+    const int x0 = t.ti * kTail, y0 = t.tj * kTail;
+    const int tx = threadIdx.x & (kTail - 1), ty = threadIdx.x / kTail;
+    double a[C], u[C], w[C];
+#pragma unroll
+    for (int r = 0; r < C; ++r) {
+      const int cl = ty + r * (256 / kTail);
+      const int x = x0 + tx, y = y0 + cl, xl = y0 + tx, yl = x0 + cl;
+      const bool in = x <= y && y < n, il = xl > yl && xl < n;   // x < n, yl < n follow
+      a[r] = in ? Tb[x + (i64)y * n] : 0.0;
+      u[r] = in ? Xb[x + (i64)y * n] : 0.0;
+      w[r] = il ? Xb[xl + (i64)yl * n] : 0.0;
+    }
+#pragma unroll
+    for (int r = 0; r < C; ++r) S[ty + r * (256 / kTail)][tx] = a[r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < C; ++r) {
+      const int cl = ty + r * (256 / kTail);
+      const int x = x0 + tx, y = y0 + cl, xl = y0 + tx, yl = x0 + cl;
+      if (x <= y && y < n) {
+        v += a[r] * a[r];
+        Xb[x + (i64)y * n] = u[r] * 1.0 + a[r] * c;
+      }
+      if (xl > yl && xl < n) {
+        const double b = herm * S[tx][cl];
+        v += b * b;
+        Tb[xl + (i64)yl * n] = b;
+        Xb[xl + (i64)yl * n] = w[r] * 1.0 + b * c;
+      }
+    }
+  } else {
+    for (int i = threadIdx.x; i < t.ti; i += 256) {
+      const double y = T[t.off + i];
+      v += y * y;
+      X[t.off + i] = X[t.off + i] * 1.0 + y * c;
+    }
+  }
+  const double s = block_sum(v, red);
+  if (threadIdx.x == 0) part[blockIdx.x] = s * t.w;
+}
+void launch_comm_tail(const DevBasis& B, const TailTask* t, int nt, double* T, int herm, double* X, double c,
+                      double* part, hipStream_t s) {
+  if (nt <= 0) return;
+  hipLaunchKernelGGL(k_comm_tail, dim3(nt, B.ninst), dim3(256), 0, s, B, t, T, herm, X, c, part);
+}
+
 // X += c * T (every element, E0 by chunk 0's first thread) and the norm
 // partials of T in the same pass: the axpy and norm of one nested
 // commutator (append_operator + mat_frob_norm, IMSRG_MAGNUS.f90:227-229),

@@ -99,6 +99,13 @@ struct GemmTask { int prob; int tm; int tn; int ks; };
 // Tile pair (I,J), I <= J, of the pppp block of channel q
 struct PairTask { int q; int ti; int tj; int pad; };
 
+// Tail of a nested commutator (k_comm_tail): tile pair (ti <= tj) of the n x n
+// square block at off, or (n = 0) ti elements from off; w: their weight in
+// the norm
+constexpr int kTail = 32;
+constexpr int kTailRun = 2048;
+struct TailTask { i64 off; int n, ti, tj, pad; double w; };
+
 // 222_ph on the grouped path: a chunk of consecutive orbit quadruples of
 // the output items (items item0 .. item0 + nitems, at most kPhChunkItems;
 // their J' terms, at most kPhChunkLanes, are gathered once into LDS)
@@ -246,6 +253,8 @@ void launch_fill_b(double* p, i64 n, double v, int ninst, const int* act, hipStr
 void launch_copy_b(double* dst, const double* src, i64 n, int ninst, const int* act, hipStream_t s);
 void launch_axpy_norm_b(const DevBasis& B, double* X, const double* T, double c, const i64* chunk_off,
                         const int* chunk_len, const double* chunk_w, int nchunk, double* part, hipStream_t s);
+void launch_comm_tail(const DevBasis& B, const TailTask* t, int nt, double* T, int herm, double* X, double c,
+                      double* part, hipStream_t s);
 void launch_norm_partials_b(const DevBasis& B, const double* op, const i64* chunk_off, const int* chunk_len,
                             const double* chunk_w, int nchunk, double* part, hipStream_t s);
 void launch_sum_sqrt_b(const DevBasis& B, const double* part, int n, double* dst, i64 sdst, int do_sqrt,
