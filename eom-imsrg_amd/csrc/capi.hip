@@ -269,14 +269,19 @@ int tiles(int n) { return (n + 63) / 64; }
 
 // Tile shapes of a basis nobody has tuned, from the number of 64 x 64 output
 // tiles of each family.  A launch of few tiles leaves CUs idle and each tile is
-// one long chain of K steps, so small families take 32 x 32 (shape 5); with
-// thousands of tiles the register-direct shapes' higher rate wins.  Measured
-// (us, every family alone, 64x64 / chosen): PPPP eMax 4 9.5 / 6.0, 5 14.9 / 8.7,
-// 6 30 / 17 (307 tiles), 7 60 / 46 (735), 8 162 / 135 (1835), 9 478 / 416; pp x
-// (ph|hh) with its epilogue eMax 5 35 / 26, 7 54 / 43, 9 173 / 151; W' eMax 5 10.3 /
-// 8.3 (294), 7 46 / 43 (2144), 8 105 / 97 (5214), 10 603 / 549 (25410).  Reverse
-// mode, whole commutator transpose: eMax 5 208 -> 185, 6 339 -> 306, 7 723 -> 687,
-// 8 unchanged.
+// one long chain of K steps, so small families take 32 x 32 (shape 5); then
+// the register-direct shapes, by 32 x 32 blocks a wave (7) and, with enough
+// tiles to fill the chip, by 64 x 32 (6; W' has too few columns to gain by it).
+// Measured (us, every family alone; shapes 5, 7, 6): PPPP eMax 4 6.2 / 6.9 / 9.2
+// (57 tiles), 5 8.9 / 8.6 / 12.6 (111), 6 16.9 / 15.4 / 19.1 (307), eMax 9 lMax 4 61 /
+// 49 / 48 (761), 8 166 / 131 / 106 (1835), 10 1866 / 1441 / 1030; pp x (ph|hh) with
+// its epilogue eMax 4 17.7 / 18.3 / 22.6 (39), 5 23.4 / 22.3 / 30.4 (59), 6 28.5 / 25.1
+// / 32.3 (151), 7 41 / 35 / 38 (387), 8 70 / 59 / 58, 10 328 / 285 / 248; W' eMax 5 8.0
+// / 8.5 / 9.8 (294), 6 18.7 / 16.2 / 16.3 (822), 8 115 / 74 / 77 (5214), 9 282 / 204 /
+// 204, 10 661 / 439 / 445 (25410).  Reverse mode, whole commutator transpose: W'
+// products (as thin as a cross-coupled block has columns, 30 - 60) shapes 5 / 7 /
+// 6 eMax 6 295 / 300 / 311, 7 681 / 666 / 687, 9 4208 / 4136 / 4168; fused pp products
+// shapes 3 / 7 / 6 eMax 6 304 / 295 / 300, 7 685 / 668 / 666, 9 4355 / 4370 / 4136.
 void default_tiles(imsrg_basis_s* B) {
   const Basis& b = B->b;
   i64 pppp = 0, ppx = 0, ph = 0;
@@ -287,13 +292,13 @@ void default_tiles(imsrg_basis_s* B) {
   }
   for (int q = 0; q < b.ncc; ++q) ph += (i64)tiles(b.rlen[q]) * (tiles(b.rlen[q]) + 1) / 2;
   const int X = IMSRG_TILE_XCD;
-  B->tile_req[0] = pppp < 512 ? 5 | X : (pppp < 1200 ? 7 | X : 6);
-  B->tile_req[1] = ppx < 700 ? 5 | X : 3 | X;
+  B->tile_req[0] = pppp < 100 ? 5 | X : (pppp < 600 ? 7 | X : 6);
+  B->tile_req[1] = ppx < 50 ? 5 | X : (ppx < 400 ? 7 | X : 6);
   B->tile_req[2] = 5 | X;
-  B->tile_req[3] = ph < 1500 ? 5 | X : (ph < 16000 ? 7 | X : 6 | X);
+  B->tile_req[3] = ph < 500 ? 5 | X : 7 | X;
   B->tile_req[4] = 5 | X;
-  B->tile_req[5] = ph < 1500 ? 5 | X : (ph < 4000 ? 7 | X : 6);
-  B->tile_req[6] = 3 | X;
+  B->tile_req[5] = ph < 1500 ? 5 | X : 7 | X;
+  B->tile_req[6] = pppp < 600 ? 7 | X : 6 | X;
 }
 
 // (re)build the tile tasks of a GEMM family for tile shape `tile`.  Groups
@@ -629,7 +634,7 @@ int build_plan(imsrg_basis_s* B) {
         p.lda = r; p.ldb = r; p.ldc = r;
         p.nprod = 2; p.ta1 = 0; p.tb1 = 1; p.ta2 = 0; p.tb2 = 1;
         p.sa1 = 0; p.sb1 = 1; p.sa2 = 1; p.sb2 = 0; p.sc = 2;
-        p.alpha = 1.0; p.s2 = 1.0; p.beta = 0.0;
+        p.alpha = 1.0; p.s2 = 1.0; p.beta = 0.0; p.upper = 1;
         B->ph.probs_h.push_back(p);
         B->ph.nks.push_back(1);
       }
@@ -1609,9 +1614,6 @@ void comm_vjp(imsrg_basis_s* B, const double* L, int Lh, const double* R, int Rh
   launch_221_vjp(D, B->one, (int)B->one_h.size(), Lh, Rh, RESb, RESh, B->Wb1, B->Wb2, s);
   Slots sp{};
   sp.p[0] = L; sp.p[1] = R; sp.p[2] = Lb; sp.p[3] = Rb; sp.p[4] = B->Wb1; sp.p[5] = B->Wb2;
-  if (B->ppb.tasks.n)
-    launch_gemm_tiled(B->ppb.tile, sp, B->ppb.probs, B->ppb.tasks.dev, B->ppb.tasks.grid, B->ppb.tasks.xmap, s,
-                      (double)Lh, (double)Rh, 1, B->ppb.sig);
   for (GemmFamily& f : B->pb)
     if (f.tasks.n) launch_gemm_tiled(f.tile, sp, f.probs, f.tasks.dev, f.tasks.grid, f.tasks.xmap, s, (double)Lh,
                                      (double)Rh, 1, f.sig);
@@ -1621,6 +1623,13 @@ void comm_vjp(imsrg_basis_s* B, const double* L, int Lh, const double* R, int Rh
   launch_122_vjp(D, B->seg_tri.dev, B->seg_tri.n, B->partners, B->partT, B->pstride, B->rowp, B->colp, B->f1off,
                  B->nf1, L, Lh, R, Rh,
                  B->cbar, RESb, RESh, Lb, Rb, s);
+  // the fused pp products last: they keep the matrix cores busy beside the end
+  // of the 222_ph chain, and the memory-bound 122 beside its gathers (eMax 8,
+  // whole transpose: 1754 us with them before the rounds, 1669 between rounds
+  // and 122, 1645 here)
+  if (B->ppb.tasks.n)
+    launch_gemm_tiled(B->ppb.tile, sp, B->ppb.probs, B->ppb.tasks.dev, B->ppb.tasks.grid, B->ppb.tasks.xmap, s,
+                      (double)Lh, (double)Rh, 1, B->ppb.sig);
   // 222_ph: the Pandya transposes of the cross-coupled cotangents (the
   // scatter transpose into the W' cotangent U and the triangular-U GEMMs ran
   // on sph)
