@@ -1,7 +1,8 @@
 // Kernels of the scalar-tensor commutator (TS_commutators.f90:10-1849) and
 // the tensor cross-coupled transform (calculate_single_pandya,
-// cross_coupled.f90:1416-1634).  One thread per two-body output element
-// (gathers, no atomics: bit-reproducible), one wave per one-body output
+// cross_coupled.f90:1416-1634).  Gathers without atomics (bit-reproducible): one
+// thread per two-body output element, or per orbit quadruple with all its
+// (J1, J2) where the terms can be shared; one wave per one-body output
 // element; the angular-momentum recouplings read host-built 6j tables.
 #include <hip/hip_runtime.h>
 
@@ -245,91 +246,37 @@ __global__ __launch_bounds__(256) void k_ts_one(DevBasis B, DevTensor T, const T
 // as a gather: the reference adds each product element Wx / Wy(IX = (d,a),
 // JX = (c,b)) of every cross-coupled block to two stored elements; here the
 // output element (P Q | Rr S; J1 J2) collects the sixteen (case, target)
-// forms it can be, with the same coefficients and the same cut |W| > 1e-6
-__device__ double ph_gather(const DevBasis& B, const DevTensor& T, const double* Wx, const double* Wy, int Lh, int Rh,
-                            int P, int Q, int Rr, int S, int J1, int J2) {
-  if ((P == Q && ((J1 >> 1) & 1)) || (Rr == S && ((J2 >> 1) & 1))) return 0.0;
-  const int R = T.rank;
-  const double thr = (double)1e-6f;
-  const int nR = R / 2 + 1;
-  double sm = 0.0;
-  for (int pat = 0; pat < 16; ++pat) {
-    int a, b, c, d;
-    bool ok;
-    switch (pat) {
-      case 0: a = P; b = Q; c = Rr; d = S; ok = true; break;                  // b>=a d>=c: (a b c d)
-      case 1: c = P; d = Q; a = Rr; b = S; ok = true; break;                  //            (c d a b)
-      case 2: a = P; b = Q; d = Rr; c = S; ok = Rr < S; break;                // b>=a d<c:  (a b d c)
-      case 3: d = P; c = Q; a = Rr; b = S; ok = P < Q; break;                 //            (d c a b)
-      case 4: b = P; a = Q; c = Rr; d = S; ok = P < Q; break;                 // b<a d>=c:  (b a c d)
-      case 5: c = P; d = Q; b = Rr; a = S; ok = Rr < S; break;                //            (c d b a)
-      case 6: b = P; a = Q; d = Rr; c = S; ok = P < Q && Rr < S; break;       // b<a d<c:   (b a d c)
-      case 7: d = P; c = Q; b = Rr; a = S; ok = P < Q && Rr < S; break;       //            (d c b a)
-      case 8: d = P; b = Q; c = Rr; a = S; ok = true; break;                  // b>=d a>=c: (d b c a)
-      case 9: c = P; a = Q; d = Rr; b = S; ok = true; break;                  //            (c a d b)
-      case 10: d = P; b = Q; a = Rr; c = S; ok = Rr < S; break;               // b>=d a<c:  (d b a c)
-      case 11: a = P; c = Q; d = Rr; b = S; ok = P < Q; break;                //            (a c d b)
-      case 12: b = P; d = Q; c = Rr; a = S; ok = P < Q; break;                // b<d a>=c:  (b d c a)
-      case 13: c = P; a = Q; b = Rr; d = S; ok = Rr < S; break;               //            (c a b d)
-      case 14: b = P; d = Q; a = Rr; c = S; ok = P < Q && Rr < S; break;      // b<d a<c:   (b d a c)
-      default: a = P; c = Q; b = Rr; d = S; ok = P < Q && Rr < S; break;      //            (a c b d)
-    }
-    if (!ok) continue;
-    const int ja = B.jj[a], jb = B.jj[b], jc = B.jj[c], jd = B.jj[d];
-    const int Tz = abs(B.tz[d] - B.tz[a]) >> 1;
-    if ((abs(B.tz[c] - B.tz[b]) >> 1) != Tz) continue;
-    const int PAR = (B.ll[d] + B.ll[a]) & 1;
-    if (((B.ll[c] + B.ll[b]) & 1) != ((PAR + (T.dpar >> 1)) & 1)) continue;
-    const double* W = pat < 8 ? Wx : Wy;
-    const double phabcd = m1pow((ja + jb + jc + jd) / 2);
-    // the J3 / J4-independent part of the pattern's coefficient; the 9j is
-    // {u1 u2 J3; u4 u5 J4; J1 J2 rank} with (u1 u2) = (ja jd) or (jd ja)
-    // and (u4 u5) = (jb jc) or (jc jb)
-    double c0;
-    bool use34;
-    switch (pat) {
-      case 0: c0 = m1pow((jb + jd + J2) / 2) * Lh; use34 = true; break;
-      case 1: c0 = -m1pow((jc + ja + J1 + R) / 2) * Rh; use34 = false; break;
-      case 2: c0 = m1pow((jb + jc) / 2) * Lh; use34 = true; break;
-      case 3: c0 = m1pow((ja - jd + R) / 2) * Rh; use34 = false; break;
-      case 4: c0 = m1pow((ja + jd + J1 + J2) / 2) * Lh; use34 = true; break;
-      case 5: c0 = m1pow((jc - jb + J1 + J2 + R) / 2) * Rh; use34 = false; break;
-      case 6: c0 = m1pow((ja + jc + J1) / 2) * Lh; use34 = true; break;
-      case 7: c0 = m1pow((jb - jd + J2 + R) / 2) * Rh; use34 = false; break;
-      case 8: c0 = m1pow((jc + ja + J2) / 2) * Lh; use34 = false; break;
-      case 9: c0 = m1pow((jd - jb + J1 + R) / 2) * Rh; use34 = true; break;
-      case 10: c0 = -Lh; use34 = false; break;
-      case 11: c0 = phabcd * m1pow(R / 2) * Rh; use34 = true; break;
-      case 12: c0 = -phabcd * m1pow((J1 + J2) / 2) * Lh; use34 = false; break;
-      case 13: c0 = m1pow((J1 + J2 + R) / 2) * Rh; use34 = true; break;
-      case 14: c0 = m1pow((jb + jd + J1) / 2) * Lh; use34 = false; break;
-      default: c0 = m1pow((ja - jc + J2 + R) / 2) * Rh; use34 = true; break;
-    }
-    const bool t2 = pat & 1;                       // the (c d a b)-type target of a case
-    const bool sw12 = (pat < 8) ? t2 : !t2;
-    const int u1 = sw12 ? jd : ja, u2 = sw12 ? ja : jd;
-    const int u4 = t2 ? jc : jb, u5 = t2 ? jb : jc;
-    double sp = 0.0;
-    for (int J3 = abs(jd - ja); J3 <= jd + ja; J3 += 2) {
-      const int IX = B.rmap[((i64)d * B.N + a) * B.nJ + (J3 >> 1)];
-      // Wy of a block with J3 = J4 is never formed (zero)
-      const int J4lo = max(max(max(abs(J3 - R), J3), abs(jc - jb)), pat < 8 ? J3 : J3 + 2);
-      const int J4hi = min(min(J3 + R, jc + jb), 2 * B.JTM);
-      for (int J4 = J4lo; J4 <= J4hi; J4 += 2) {
-        const i64* wt = T.wtab + ((((J3 >> 1) * nR + ((J4 - J3) >> 1)) << 2) + 2 * Tz + PAR) * 2;
-        const int JX = B.rmap[((i64)c * B.N + b) * B.nJ + (J4 >> 1)];
-        const double w = W[wt[0] + IX + JX * wt[1]];
-        if (!(fabs(w) > thr)) continue;
-        const double v = n9(T, u1, u2, J3, u4, u5, J4, J1, J2) * w;
-        sp += (use34 && (((J3 + J4) >> 1) & 1)) ? -v : v;
-      }
-    }
-    sm += c0 * sp;
+// forms it can be, with the same coefficients and the same cut |W| > 1e-6:
+//    0 (a b c d)   1 (c d a b)   2 (a b d c)   3 (d c a b)     Wx, b>=a d>=c | b>=a d<c
+//    4 (b a c d)   5 (c d b a)   6 (b a d c)   7 (d c b a)     Wx, b<a d>=c  | b<a d<c
+//    8 (d b c a)   9 (c a d b)  10 (d b a c)  11 (a c d b)     Wy, b>=d a>=c | b>=d a<c
+//   12 (b d c a)  13 (c a b d)  14 (b d a c)  15 (a c b d)     Wy, b<d a>=c  | b<d a<c
+// kPatPos: per pattern, the places (0 P, 1 Q, 2 Rr, 3 S) of a, b, c, d, two
+// bits each; a pattern in kPatBra needs P < Q, in kPatKet Rr < S (tensor.hpp).
+// J3 / J4-independent part of a pattern's coefficient
+__device__ __forceinline__ double ts_pat_coef(int pat, int ja, int jb, int jc, int jd, int J1, int J2, int R, int Lh,
+                                              int Rh) {
+  const int all = (ja + jb + jc + jd) / 2;
+  int e, s;
+  switch (pat) {
+    case 0: e = (jb + jd + J2) / 2; s = Lh; break;
+    case 1: e = (jc + ja + J1 + R) / 2; s = -Rh; break;
+    case 2: e = (jb + jc) / 2; s = Lh; break;
+    case 3: e = (ja - jd + R) / 2; s = Rh; break;
+    case 4: e = (ja + jd + J1 + J2) / 2; s = Lh; break;
+    case 5: e = (jc - jb + J1 + J2 + R) / 2; s = Rh; break;
+    case 6: e = (ja + jc + J1) / 2; s = Lh; break;
+    case 7: e = (jb - jd + J2 + R) / 2; s = Rh; break;
+    case 8: e = (jc + ja + J2) / 2; s = Lh; break;
+    case 9: e = (jd - jb + J1 + R) / 2; s = Rh; break;
+    case 10: e = 0; s = -Lh; break;
+    case 11: e = all + R / 2; s = Rh; break;
+    case 12: e = all + (J1 + J2) / 2; s = -Lh; break;
+    case 13: e = (J1 + J2 + R) / 2; s = Rh; break;
+    case 14: e = (jb + jd + J1) / 2; s = Lh; break;
+    default: e = (ja - jc + J2 + R) / 2; s = Rh; break;
   }
-  sm *= sqrt((J1 + 1.0) * (J2 + 1.0));
-  if (P == Q) sm *= 1.4142135623730951;
-  if (Rr == S) sm *= 1.4142135623730951;
-  return sm;
+  return (double)(m1pow(e) * s);
 }
 
 // TS_commutator_122 of one output element (TS_commutators.f90:555-663)
@@ -357,35 +304,6 @@ __device__ double ts122(const DevBasis& B, const DevTensor& T, const double* L, 
   return sm;
 }
 
-// TS_commutator_212 of one output element (TS_commutators.f90:666-806)
-__device__ double ts212(const DevBasis& B, const DevTensor& T, const double* L, int Lh, const double* R, int Rh, int a,
-                        int b, int c, int d, int J1, int J2) {
-  const int rank = T.rank;
-  const int ja = B.jj[a], jb = B.jj[b], jc = B.jj[c], jd = B.jj[d];
-  const int ta = B.tz[a], tb = B.tz[b], tc = B.tz[c], td = B.tz[d];
-  const int mla = B.ll[a] & 1, mlb = B.ll[b] & 1, mlc = B.ll[c] & 1, mld = B.ll[d] & 1;
-  double sm = 0.0;
-  for (int i = 0; i < B.N; ++i) {
-    const int ji = B.jj[i], ti = B.tz[i], mli = (B.ll[i] + (T.dpar >> 1)) & 1;
-    double s1 = 0.0, s2 = 0.0, s3 = 0.0, s4 = 0.0;
-    if (ti == ta && mli == mla && dtri(ji, ja, rank))
-      s1 = -x6(T, J1, J2, ji, ja, jb) * f_tensor_elem(B, R, Rh, a, i) * v_elem(B, L, Lh, i, b, c, d, J2);
-    s1 = s1 * m1pow((ja + jb - J2) / 2);
-    if (ti == tb && mli == mlb && dtri(ji, jb, rank))
-      s2 = x6(T, J1, J2, ji, jb, ja) * f_tensor_elem(B, R, Rh, b, i) * v_elem(B, L, Lh, i, a, c, d, J2);
-    s2 = s2 * m1pow((J1 + J2) / 2);
-    if (ti == td && mli == mld && dtri(ji, jd, rank))
-      s3 = x6(T, J1, J2, jd, ji, jc) * f_tensor_elem(B, R, Rh, i, d) * v_elem(B, L, Lh, a, b, c, i, J1);
-    s3 = s3 * m1pow((jc + jd - J1) / 2);
-    if (ti == tc && mli == mlc && dtri(ji, jc, rank))
-      s4 = -x6(T, J1, J2, jc, ji, jd) * f_tensor_elem(B, R, Rh, i, c) * v_elem(B, L, Lh, a, b, d, i, J1);
-    s4 = s4 * m1pow((J2 + J1) / 2);
-    sm = sm + (s1 + s2 + s3 + s4);
-  }
-  sm = sm * sqrt((J1 + 1.0) * (J2 + 1.0) / (1.0 + (a == b)) / (1.0 + (c == d))) * m1pow(rank / 2);
-  return sm;
-}
-
 // TS_commutator_122 (assigns), one thread per stored two-body element in
 // tiles of 256 consecutive elements of a sub-block
 __global__ __launch_bounds__(256) void k_ts122(DevBasis B, DevTensor T, const TSub* subs, const TElem* tasks,
@@ -402,31 +320,187 @@ __global__ __launch_bounds__(256) void k_ts122(DevBasis B, DevTensor T, const TS
   RES[sb.off + IX + (i64)JX * sb.n1] = ts122(B, T, L, Lh, R, Rh, a, b, c, d, J1, J2);
 }
 
-// TS_commutator_212 (adds), one thread per element of the quadruple-ordered
-// output list (neighbouring lanes share the orbit quadruple and so the orbit
-// loop and its conditions)
-__global__ __launch_bounds__(256) void k_ts212(DevBasis B, DevTensor T, const TPh* tasks, i64 nt, const double* L,
-                                               int Lh, const double* R, int Rh, double* RES) {
-  const i64 e = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= nt) return;
-  const TPh t = tasks[e];
-  const int u = t.abcd;
-  RES[t.off] += ts212(B, T, L, Lh, R, Rh, u & 255, (u >> 8) & 255, (u >> 16) & 255, (u >> 24) & 255, t.jj & 0xffff,
-                      t.jj >> 16);
+// TS_commutator_212 (TS_commutators.f90:666-806; adds), one wave per pack of
+// orbit quadruples that share their four j: of
+//   sum_i f(a i) v(i b c d; J2), f(b i) v(i a c d; J2),
+//   sum_i f(i d) v(a b c i; J1), f(i c) v(a b d i; J1)
+// a lane forms each product once for all outputs (J1, J2) of its quadruple,
+// the 6j coefficients come from LDS as broadcasts, and i runs over the
+// partners of its orbit by their j.  The address unit (uncoalesced element
+// and pair-number reads) bounds it.  One thread per output, every orbit
+// tested: 10.5 -> 5.0 ms; over the partners only 9.7 (eMax 8, rank 4).
+__global__ __launch_bounds__(64) void k_ts212(DevBasis B, DevTensor T, const TPh* tasks, const TPack* packs,
+                                              const int2* quads, const double* L, int Lh, const double* R, int Rh,
+                                              double* RES) {
+  __shared__ double cf[kTsRows * kTsOut];
+  const int lane = threadIdx.x;
+  const TPack p = packs[blockIdx.x];
+  const int rank = T.rank, N = B.N, nJ = B.nJ, nr = rank + 1;
+  const int2 mine = quads[p.q0 + min(lane, p.nq - 1)], first = quads[p.q0];
+  const int u = mine.x, u0 = __builtin_amdgcn_readfirstlane(first.x), f0 = __builtin_amdgcn_readfirstlane(first.y);
+  const bool eqb = (u0 & 255) == ((u0 >> 8) & 255), eqk = ((u0 >> 16) & 255) == ((u0 >> 24) & 255);
+  int j0[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) j0[k] = B.jj[(u0 >> (8 * k)) & 255];
+  for (int ob = 0; ob < p.no; ob += kTsOut) {
+    double acc[kTsOut];
+#pragma unroll
+    for (int o = 0; o < kTsOut; ++o) acc[o] = 0.0;
+    // side 0: partners of a, v(i b c d); 1: of b, v(i a c d); 2: of d, v(a b c i);
+    // 3: of c, v(a b d i)
+    for (int sd = 0; sd < 4; ++sd) {
+      const bool bra = sd < 2;
+      const int kx = sd == 0 ? 0 : (sd == 1 ? 1 : (sd == 2 ? 3 : 2)), ky = kx ^ 1;
+      const int x = (u >> (8 * kx)) & 255, y = (u >> (8 * ky)) & 255;               // i's orbit, its pair partner
+      const int e0 = (u >> (bra ? 16 : 0)) & 255, e1 = (u >> (bra ? 24 : 8)) & 255;   // the other pair
+      const int jx = j0[kx], jy = j0[ky], je0 = j0[bra ? 2 : 0], je1 = j0[bra ? 3 : 1];
+      const int cx = B.con[x], cy = B.con[y], ce = B.con[e0] + B.con[e1];
+      const int q0 = 2 * ((B.tz[e0] + B.tz[e1]) / 2 + 1) + ((B.ll[e0] + B.ll[e1]) & 1);
+      for (int ji = max(1, jx - rank); ji <= jx + rank; ji += 2) {
+        const int jr = (ji - jx + rank) / 2;
+        if (ji + jx < rank) continue;
+        const int Jlo = max(abs(ji - jy), abs(je0 - je1)), Jhi = min(ji + jy, je0 + je1);
+        const int s0 = T.fst[x * nr + jr], n = T.fst[x * nr + jr + 1] - s0;
+        for (int Ja = Jlo; Ja <= Jhi; Ja += 2 * kTsRows) {
+          const int Je = min(Jhi, Ja + 2 * kTsRows - 2);
+          __syncthreads();
+          for (int t = lane; t < ((Je - Ja) / 2 + 1) * kTsOut; t += 64) {
+            const int J = Ja + 2 * (t / kTsOut), o = ob + (t & (kTsOut - 1));
+            double c = 0.0;
+            if (o < p.no) {
+              const int jj = tasks[f0 + o].jj, J1 = jj & 0xffff, J2 = jj >> 16;
+              if ((bra ? J2 : J1) == J) {
+                if (sd == 0) c = -x6(T, J1, J2, ji, jx, jy) * m1pow((jx + jy - J2) / 2);
+                else if (sd == 1) c = x6(T, J1, J2, ji, jx, jy) * m1pow((J1 + J2) / 2);
+                else if (sd == 2) c = x6(T, J1, J2, jx, ji, jy) * m1pow((jx + jy - J1) / 2);
+                else c = -x6(T, J1, J2, jx, ji, jy) * m1pow((J1 + J2) / 2);
+              }
+            }
+            cf[t] = c;
+          }
+          __syncthreads();
+          for (int k = 0; k < n; ++k) {
+            const int i = T.fmem[s0 + k], ci = B.con[i];
+            const double f = bra ? f_tensor_elem(B, R, Rh, x, i) : f_tensor_elem(B, R, Rh, i, x);
+            // <i y | e> or <e | y i>
+            const int c1 = bra ? ci + cy : ce, c2 = bra ? ce : ci + cy;
+            const int lo = min(c1, c2), hi = max(c1, c2), g = blk_of(lo, hi);
+            double ph0 = e0 == e1 ? 1.4142135623730951 : 1.0;
+            const int pi = i < y ? i * N + y : y * N + i;
+            const bool sw = bra ? i > y : y > i;          // stored in the other order
+            if (i == y) ph0 *= 1.4142135623730951;
+            const int* mi = B.xmap + (i64)pi * nJ;
+            const int* me = B.xmap + ((i64)e0 * N + e1) * nJ;
+            if (c1 > c2) ph0 *= Lh;
+#pragma unroll 2
+            for (int J = Ja; J <= Je; J += 2) {
+              const int q = 3 * J + q0;
+              const int a1 = mi[J >> 1], a2 = me[J >> 1];
+              const int row = (c1 > c2) == bra ? a2 : a1, col = (c1 > c2) == bra ? a1 : a2;
+              double v = L[B.goff[q * 6 + g] + row + (i64)col * B.dims[q * 3 + lo]];
+              v *= (sw && !(((ji + jy - J) >> 1) & 1)) ? -ph0 : ph0;   // (-1)^(1 + (ji + jy - J) / 2)
+              const double w = f * v;
+              const double* c = cf + ((J - Ja) >> 1) * kTsOut;
+#pragma unroll
+              for (int o = 0; o < kTsOut; ++o) acc[o] = fma(c[o], w, acc[o]);
+            }
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int o = 0; o < kTsOut; ++o)
+      if (ob + o < p.no && lane < p.nq) {
+        const TPh t = tasks[mine.y + ob + o];
+        RES[t.off] += acc[o] * (sqrt(((t.jj & 0xffff) + 1.0) * ((t.jj >> 16) + 1.0) / (1.0 + eqb) / (1.0 + eqk)) *
+                                m1pow(rank / 2));
+      }
+  }
 }
 
-// the 222_ph back-transform, one thread per output element of the
-// quadruple-ordered list: neighbouring lanes share the orbit quadruple, so
-// they run the same pattern and (J3, J4) loops and read the same W elements
-// and one run of 9j symbols
-__global__ __launch_bounds__(256) void k_ts_ph(DevBasis B, DevTensor T, const TPh* tasks, i64 nt, int Lh, int Rh,
-                                               const double* Wx, const double* Wy, double* RES) {
-  const i64 e = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= nt) return;
-  const TPh t = tasks[e];
-  const int u = t.abcd;
-  RES[t.off] += ph_gather(B, T, Wx, Wy, Lh, Rh, u & 255, (u >> 8) & 255, (u >> 16) & 255, (u >> 24) & 255,
-                          t.jj & 0xffff, t.jj >> 16);
+// The 222_ph back-transform, one wave per pack of orbit quadruples that share
+// their four j, their patterns and so every (J3, J4) loop and every 9j symbol:
+// a lane holds one quadruple and gathers its W elements once for kTsOut
+// outputs (J1, J2); the coefficients of a pattern (9j, signs) are staged in
+// LDS once for the wave and read as broadcasts.  Gathers of W and of its row
+// numbers bound it.  One thread per output, which walks every term's loads
+// by itself and diverges between quadruples: 16.8 -> 5.5 ms (eMax 8, rank 4;
+// 8 outputs at a time 7.9, 32 8.2).
+__global__ __launch_bounds__(64) void k_ts_ph(DevBasis B, DevTensor T, const TPh* tasks, const TPack* packs,
+                                              const int2* quads, int Lh, int Rh, const double* Wx, const double* Wy,
+                                              double* RES) {
+  __shared__ double cf[kTsRows * kTsOut];
+  const int lane = threadIdx.x;
+  const TPack p = packs[blockIdx.x];
+  const int R = T.rank, nR = R / 2 + 1, nE = min(nR, T.nJ), N = B.N, nJ = B.nJ, J4max = 2 * B.JTM;
+  const double thr = (double)1e-6f;
+  const int2 mine = quads[p.q0 + min(lane, p.nq - 1)], first = quads[p.q0];
+  const int u = mine.x, u0 = __builtin_amdgcn_readfirstlane(first.x), f0 = __builtin_amdgcn_readfirstlane(first.y);
+  const bool eqb = (u0 & 255) == ((u0 >> 8) & 255), eqk = ((u0 >> 16) & 255) == ((u0 >> 24) & 255);
+  for (int ob = 0; ob < p.no; ob += kTsOut) {
+    double acc[kTsOut];
+#pragma unroll
+    for (int o = 0; o < kTsOut; ++o) acc[o] = 0.0;
+    for (unsigned m = p.mask; m; m &= m - 1) {
+      const int pat = __builtin_ctz(m);
+      const TPat x0 = ts_pat(pat, u0), x = ts_pat(pat, u);
+      const int ja = B.jj[x0.a], jb = B.jj[x0.b], jc = B.jj[x0.c], jd = B.jj[x0.d];   // of every lane
+      const int wsel = 2 * (abs(B.tz[x.d] - B.tz[x.a]) >> 1) + ((B.ll[x.d] + B.ll[x.a]) & 1);
+      const int* rx = B.rmap + ((i64)x.d * N + x.a) * nJ;
+      const int* ry = B.rmap + ((i64)x.c * N + x.b) * nJ;
+      const double* W = pat < 8 ? Wx : Wy;
+      // the 9j is {u1 u2 J3; u4 u5 J4; J1 J2 rank}, (u1 u2) = (ja jd) or (jd ja),
+      // (u4 u5) = (jb jc) or (jc jb)
+      const bool t2 = pat & 1, sw12 = (pat < 8) ? t2 : !t2;
+      const int u1 = sw12 ? jd : ja, u2 = sw12 ? ja : jd, u4 = t2 ? jc : jb, u5 = t2 ? jb : jc;
+      const double* n9 = T.n9 + ((((i64)(u1 >> 1) * T.nho + (u2 >> 1)) * T.nho + (u4 >> 1)) * T.nho + (u5 >> 1)) * T.nJ *
+                                    nR * T.nJ * nR;
+      // Wy of a block with J3 = J4 is never formed (zero)
+      const int k0 = pat < 8 ? 0 : 1, Jmn = abs(jc - jb), Jmx = min(jc + jb, J4max);
+      const int JC = 2 * (kTsRows / nE);
+      for (int Ja = abs(jd - ja); Ja <= jd + ja; Ja += JC) {
+        const int Je = min(jd + ja, Ja + JC - 2), rows = ((Je - Ja) / 2 + 1) * nE;
+        __syncthreads();
+        for (int t = lane; t < rows * kTsOut; t += 64) {
+          const int r = t / kTsOut, o = ob + (t & (kTsOut - 1)), j = r / nE, k = r - j * nE;
+          const int J3 = Ja + 2 * j, J4 = J3 + 2 * k;
+          double c = 0.0;
+          if (o < p.no && J4 <= Jmx) {
+            const int jj = tasks[f0 + o].jj, J1 = jj & 0xffff, J2 = jj >> 16;
+            if (!((eqb && ((J1 >> 1) & 1)) || (eqk && ((J2 >> 1) & 1)))) {
+              c = n9[(((i64)(J3 >> 1) * nR + k) * T.nJ + (J1 >> 1)) * nR + ((J2 - J1) >> 1)] *
+                  ts_pat_coef(pat, ja, jb, jc, jd, J1, J2, R, Lh, Rh);
+              if (((kPat34 >> pat) & 1) && (((J3 + J4) >> 1) & 1)) c = -c;
+            }
+          }
+          cf[t] = c;
+        }
+        __syncthreads();
+        for (int J3 = Ja; J3 <= Je; J3 += 2) {
+          const int IX = rx[J3 >> 1];
+          const int ke = min(nE - 1, (Jmx - J3) >> 1);
+          const double* c = cf + ((J3 - Ja) >> 1) * nE * kTsOut;
+#pragma unroll 3
+          for (int k = max(k0, (max(R - J3, Jmn) - J3 + 1) >> 1); k <= ke; ++k) {
+            const i64* wt = T.wtab + ((((J3 >> 1) * nR + k) << 2) + wsel) * 2;
+            const double v = W[wt[0] + IX + ry[(J3 >> 1) + k] * wt[1]];
+            const double w = fabs(v) > thr ? v : 0.0;
+#pragma unroll
+            for (int o = 0; o < kTsOut; ++o) acc[o] = fma(c[k * kTsOut + o], w, acc[o]);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int o = 0; o < kTsOut; ++o)
+      if (ob + o < p.no && lane < p.nq) {
+        const TPh t = tasks[mine.y + ob + o];
+        double sm = acc[o] * sqrt(((t.jj & 0xffff) + 1.0) * ((t.jj >> 16) + 1.0));
+        if (eqb) sm *= 1.4142135623730951;
+        if (eqk) sm *= 1.4142135623730951;
+        RES[t.off] += sm;
+      }
+  }
 }
 
 // calculate_single_pandya, cross_coupled.f90:1416-1634, one thread per
@@ -539,19 +613,15 @@ void launch_ts122(const DevBasis& B, const DevTensor& T, const TSub* sb, const T
   if (nt > 0) hipLaunchKernelGGL(k_ts122, dim3(nt), dim3(256), 0, s, B, T, sb, t, L, Lh, R, Rh, RES);
 }
 
-void launch_ts212(const DevBasis& B, const DevTensor& T, const TPh* t, i64 nt, const double* L, int Lh,
-                  const double* R, int Rh, double* RES, hipStream_t s) {
-  if (nt > 0)
-    hipLaunchKernelGGL(k_ts212, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, s, B, T, t, nt, L, Lh, R, Rh, RES);
+void launch_ts212(const DevBasis& B, const DevTensor& T, const TPh* t, const TPack* p, int np, const int2* q,
+                  const double* L, int Lh, const double* R, int Rh, double* RES, hipStream_t s) {
+  if (np > 0) hipLaunchKernelGGL(k_ts212, dim3(np), dim3(64), 0, s, B, T, t, p, q, L, Lh, R, Rh, RES);
 }
 
-void launch_ts_ph(const DevBasis& B, const DevTensor& T, const TPh* t, i64 nt, int Lh, int Rh, const double* Wx,
-                  const double* Wy, double* RES, hipStream_t s) {
-  if (nt > 0)
-    hipLaunchKernelGGL(k_ts_ph, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, s, B, T, t, nt, Lh, Rh, Wx, Wy,
-                       RES);
+void launch_ts_ph(const DevBasis& B, const DevTensor& T, const TPh* t, const TPack* p, int np, const int2* q, int Lh,
+                  int Rh, const double* Wx, const double* Wy, double* RES, hipStream_t s) {
+  if (np > 0) hipLaunchKernelGGL(k_ts_ph, dim3(np), dim3(64), 0, s, B, T, t, p, q, Lh, Rh, Wx, Wy, RES);
 }
-
 void launch_ts_pandya(const DevBasis& B, const DevTensor& T, const TCC* t, int nt, const double* R, int Rh,
                       double* CC, hipStream_t s) {
   if (nt) hipLaunchKernelGGL(k_ts_pandya, dim3(nt), dim3(256), 0, s, B, T, t, R, Rh, CC);

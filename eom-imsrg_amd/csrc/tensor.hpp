@@ -40,6 +40,8 @@ struct DevTensor {
                                    // 222_ph back-transform, J3 <= J4 <= J3 + rank, J1 <= J2 <= J1 + rank:
                                    // [u1/2][u2/2][u4/2][u5/2][J3/2][(J4-J3)/2][J1/2][(J2-J1)/2]
                                    // (the outputs of one orbit quadruple read one contiguous run)
+  const int *fst, *fmem;           // orbits of 2j = 2j_x - rank + 2r that a rank / dpar one-body operator couples
+                                   // to orbit x: fmem[fst[k]] .. fmem[fst[k + 1] - 1], k = x (rank + 1) + r
   int nJ, nhx, nho;                // 2J/2 values; half-integers up to jmax + rank; up to jmax
 };
 
@@ -51,6 +53,37 @@ struct TElem { int sb; int start; };
 // (a | b << 8 | c << 16 | d << 24) and 2J1 | 2J2 << 16; the list is ordered
 // by orbit quadruple, so the lanes of a wave share the quadruple's loops
 struct TPh { int off, abcd, jj; };
+// at most 64 quadruples of that list (quads q0 .. q0 + nq: orbits, first
+// output) with the same four j, patterns and outputs (J1, J2)
+struct TPack { int q0, nq, no; unsigned mask; };
+constexpr int kTsOut = 16;    // outputs a lane accumulates at a time
+constexpr int kTsRows = 64;   // (J3, J4) pairs whose coefficients are staged at a time
+
+// The sixteen (case, target) forms of 222_ph's back-transform (tensor.hip):
+// places of a, b, c, d among the output's orbits, and what a form needs
+constexpr unsigned pos4(int a, int b, int c, int d) { return a | (b << 2) | (c << 4) | (d << 6); }
+constexpr unsigned long long pos8(unsigned a, unsigned b, unsigned c, unsigned d, unsigned e, unsigned f, unsigned g,
+                                  unsigned h) {
+  return (unsigned long long)(a | (b << 8) | (c << 16) | (d << 24)) |
+         ((unsigned long long)(e | (f << 8) | (g << 16) | (h << 24)) << 32);
+}
+constexpr unsigned long long kPatPos0 = pos8(pos4(0, 1, 2, 3), pos4(2, 3, 0, 1), pos4(0, 1, 3, 2), pos4(2, 3, 1, 0),
+                                             pos4(1, 0, 2, 3), pos4(3, 2, 0, 1), pos4(1, 0, 3, 2), pos4(3, 2, 1, 0));
+constexpr unsigned long long kPatPos1 = pos8(pos4(3, 1, 2, 0), pos4(1, 3, 0, 2), pos4(2, 1, 3, 0), pos4(0, 3, 1, 2),
+                                             pos4(3, 0, 2, 1), pos4(1, 2, 0, 3), pos4(2, 0, 3, 1), pos4(0, 2, 1, 3));
+constexpr unsigned kPatBra = 0xd8d8, kPatKet = 0xe4e4, kPat34 = 0xaa55;   // kPat34: sign (-1)^((J3+J4)/2)
+
+struct TPat { int a, b, c, d; };
+__host__ __device__ inline TPat ts_pat(int pat, int u) {
+  const unsigned m = (unsigned)((pat < 8 ? kPatPos0 : kPatPos1) >> (8 * (pat & 7))) & 255;
+  TPat x;
+  x.a = (u >> (8 * (m & 3))) & 255;
+  x.b = (u >> (8 * ((m >> 2) & 3))) & 255;
+  x.c = (u >> (8 * ((m >> 4) & 3))) & 255;
+  x.d = (u >> (8 * ((m >> 6) & 3))) & 255;
+  return x;
+}
+
 // one-body output: cls 0 fhh (p <= q, mirrored), 1 fpp (p <= q, mirrored), 2 fph
 struct TOne { int cls, p, q, pad; };
 // 256 consecutive elements of CCX (term 1) or CCR (term 2) of block qx
@@ -65,13 +98,12 @@ void launch_ts_one(int mode, const DevBasis& B, const DevTensor& T, const TOne* 
 // TS_commutator_122 (assigns) over element tiles
 void launch_ts122(const DevBasis& B, const DevTensor& T, const TSub* sb, const TElem* t, int nt, const double* L,
                   int Lh, const double* R, int Rh, double* RES, hipStream_t s);
-// TS_commutator_212 (adds) over the quadruple-ordered output list
-void launch_ts212(const DevBasis& B, const DevTensor& T, const TPh* t, i64 nt, const double* L, int Lh,
-                  const double* R, int Rh, double* RES, hipStream_t s);
-// the back-transform of TS_commutator_222_ph from the products Wx / Wy, one
-// thread per listed output element
-void launch_ts_ph(const DevBasis& B, const DevTensor& T, const TPh* t, i64 nt, int Lh, int Rh, const double* Wx,
-                  const double* Wy, double* RES, hipStream_t s);
+// TS_commutator_212 (adds)
+void launch_ts212(const DevBasis& B, const DevTensor& T, const TPh* t, const TPack* p, int np, const int2* q,
+                  const double* L, int Lh, const double* R, int Rh, double* RES, hipStream_t s);
+// the back-transform of TS_commutator_222_ph from the products Wx / Wy
+void launch_ts_ph(const DevBasis& B, const DevTensor& T, const TPh* t, const TPack* p, int np, const int2* q, int Lh,
+                  int Rh, const double* Wx, const double* Wy, double* RES, hipStream_t s);
 // calculate_single_pandya of every listed (block, term) into CC
 void launch_ts_pandya(const DevBasis& B, const DevTensor& T, const TCC* t, int nt, const double* R, int Rh,
                       double* CC, hipStream_t s);
