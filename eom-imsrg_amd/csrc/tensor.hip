@@ -279,33 +279,43 @@ __device__ __forceinline__ double ts_pat_coef(int pat, int ja, int jb, int jc, i
   return (double)(m1pow(e) * s);
 }
 
-// TS_commutator_122 of one output element (TS_commutators.f90:555-663)
-__device__ double ts122(const DevBasis& B, const DevTensor& T, const double* L, int Lh, const double* R, int Rh, int a,
-                        int b, int c, int d, int J1, int J2) {
-  double sm = 0.0;
-  const int sa = B.spblk[a], sbk = B.spblk[b], sc = B.spblk[c], sd = B.spblk[d];
-  for (int k = B.spstart[sa]; k < B.spstart[sa + 1]; ++k) {
-    const int i = B.spmem[k];
-    sm = sm + f_elem(B, L, Lh, a, i) * tensor_elem(B, T, R, Rh, i, b, c, d, J1, J2);
-  }
-  for (int k = B.spstart[sbk]; k < B.spstart[sbk + 1]; ++k) {
-    const int i = B.spmem[k];
-    sm = sm + f_elem(B, L, Lh, b, i) * tensor_elem(B, T, R, Rh, a, i, c, d, J1, J2);
-  }
-  for (int k = B.spstart[sc]; k < B.spstart[sc + 1]; ++k) {
-    const int i = B.spmem[k];
-    sm = sm - f_elem(B, L, Lh, i, c) * tensor_elem(B, T, R, Rh, a, b, i, d, J1, J2);
-  }
-  for (int k = B.spstart[sd]; k < B.spstart[sd + 1]; ++k) {
-    const int i = B.spmem[k];
-    sm = sm - f_elem(B, L, Lh, i, d) * tensor_elem(B, T, R, Rh, a, b, c, i, J1, J2);
-  }
-  sm = sm / sqrt(1.0 + (a == b)) / sqrt(1.0 + (c == d));
-  return sm;
+// TS_commutator_122 of one output element (TS_commutators.f90:555-663) of
+// block q, row pair (a, b) number IX and column pair (c, d) number JX of their
+// classes.  A partner i of a keeps (l, j, tz), so the element <i b | c d> is in
+// the same block: only its row number and sub-block change.
+__device__ double ts122(const DevBasis& B, const DevTensor& T, const double* L, int Lh, const double* R, int q, int IX,
+                        int JX, int a, int b, int c, int d, int J1, int J2) {
+  const int N = B.N, C1 = B.con[a] + B.con[b] + 1, C2 = B.con[c] + B.con[d] + 1;
+  const i64* goff = T.tgoff + q * 9;
+  const int* dim = T.tdim + q * 6;
+  auto sum = [&](int x, int y, bool bra, bool first) {   // partners of x, the first / second of its pair with y
+    const int J = bra ? J1 : J2, sx = B.spblk[x], cy = B.con[y];
+    const int odd = ((B.jj[x] + B.jj[y] - J) >> 1) & 1;
+    double sm = 0.0;
+    for (int k = B.spstart[sx]; k < B.spstart[sx + 1]; ++k) {
+      const int i = B.spmem[k], Ci = B.con[i] + cy + 1;
+      const int g = bra ? tsub(Ci, C2) : tsub(C1, Ci);
+      const int n = B.xmap[((i64)i * N + y) * B.nJ + (J >> 1)];
+      const double v = R[goff[g] + (bra ? n : IX) + (i64)(bra ? JX : n) * dim[kTSea1[g]]];
+      // pairs are stored in orbit order: (-1)^(1 + (jx + jy - J) / 2) for the other
+      const bool sw = first ? i > y : y > i;
+      const double pre = i == y ? 1.4142135623730951 : (sw && !odd ? -1.0 : 1.0);
+      sm = sm + (bra ? f_elem(B, L, Lh, x, i) : f_elem(B, L, Lh, i, x)) * (v * pre);
+    }
+    return sm;
+  };
+  const double e1 = a == b ? 1.4142135623730951 : 1.0, e2 = c == d ? 1.4142135623730951 : 1.0;
+  double sm = sum(a, b, true, true) * e2;
+  sm = sm + sum(b, a, true, false) * e2;
+  sm = sm - sum(c, d, false, true) * e1;
+  sm = sm - sum(d, c, false, false) * e1;
+  return sm / e1 / e2;
 }
 
 // TS_commutator_122 (assigns), one thread per stored two-body element in
-// tiles of 256 consecutive elements of a sub-block
+// tiles of 256 consecutive elements of a sub-block.  Looking every element up
+// from its four orbits took 2.6 ms, its place in the known block 1.3 (eMax 8,
+// rank 4).
 __global__ __launch_bounds__(256) void k_ts122(DevBasis B, DevTensor T, const TSub* subs, const TElem* tasks,
                                                const double* L, int Lh, const double* R, int Rh, double* RES) {
   const TElem t = tasks[blockIdx.x];
@@ -317,7 +327,7 @@ __global__ __launch_bounds__(256) void k_ts122(DevBasis B, DevTensor T, const TS
   unpack(B.pairs[sb.roff + IX], a, b);
   unpack(B.pairs[sb.coff + JX], c, d);
   const int J1 = T.blk[sb.q * 8], J2 = T.blk[sb.q * 8 + 1];
-  RES[sb.off + IX + (i64)JX * sb.n1] = ts122(B, T, L, Lh, R, Rh, a, b, c, d, J1, J2);
+  RES[sb.off + IX + (i64)JX * sb.n1] = ts122(B, T, L, Lh, R, sb.q, IX, JX, a, b, c, d, J1, J2);
 }
 
 // TS_commutator_212 (TS_commutators.f90:666-806; adds), one wave per pack of
@@ -505,6 +515,8 @@ __global__ __launch_bounds__(64) void k_ts_ph(DevBasis B, DevTensor T, const TPh
 
 // calculate_single_pandya, cross_coupled.f90:1416-1634, one thread per
 // element of CCX(qx) (term 1: r1 x nb2) or CCR(qx) (term 2: nb1 x r2)
+// J4 runs only where the tensor couples it to J3 (over its whole range, with a
+// 9j for each, 1.02 -> 0.72 ms a launch at eMax 8, rank 4).
 __global__ __launch_bounds__(256) void k_ts_pandya(DevBasis B, DevTensor T, const TCC* tasks, const double* R, int Rh,
                                                    double* CC) {
   const TCC t = tasks[blockIdx.x];
@@ -527,7 +539,7 @@ __global__ __launch_bounds__(256) void k_ts_pandya(DevBasis B, DevTensor T, cons
     if (cons) {
       const int ja = B.jj[a], jb = B.jj[b], jp = B.jj[p], jh = B.jj[h];
       for (int J3 = abs(ja - jh); J3 <= ja + jh; J3 += 2)
-        for (int J4 = abs(jp - jb); J4 <= jp + jb; J4 += 2)
+        for (int J4 = max(abs(jp - jb), abs(J3 - T.rank)); J4 <= min(jp + jb, J3 + T.rank); J4 += 2)
           sm = sm - m1pow(J4 / 2) * sqrt((J3 + 1.0) * (J4 + 1.0)) * ninej(T, ja, jb, J3c, jh, jp, J4c, J3, J4) *
                         tensor_elem(B, T, R, Rh, a, h, p, b, J3, J4);
       sm = sm * m1pow((jh + jb + J4c) / 2) * sqrt((J3c + 1.0) * (J4c + 1.0));
@@ -545,7 +557,7 @@ __global__ __launch_bounds__(256) void k_ts_pandya(DevBasis B, DevTensor T, cons
     if (cons) {
       const int ja = B.jj[a], jb = B.jj[b], jp = B.jj[p], jh = B.jj[h];
       for (int J3 = abs(ja - jh); J3 <= ja + jh; J3 += 2)
-        for (int J4 = abs(jp - jb); J4 <= jp + jb; J4 += 2)
+        for (int J4 = max(abs(jp - jb), abs(J3 - T.rank)); J4 <= min(jp + jb, J3 + T.rank); J4 += 2)
           sm = sm - m1pow(J4 / 2) * sqrt((J3 + 1.0) * (J4 + 1.0)) * ninej(T, jh, jp, J3c, ja, jb, J4c, J3, J4) *
                         tensor_elem(B, T, R, Rh, h, a, b, p, J3, J4);
       sm = sm * m1pow((jp + ja + J4c) / 2) * sqrt((J3c + 1.0) * (J4c + 1.0)) * m1pow((jp + jh) / 2);
