@@ -1045,16 +1045,19 @@ __device__ __forceinline__ void d_comm121(DevBasis B, const OneTask* tasks, cons
   if (threadIdx.x == 0) onebody_update(B, t, sm / (B.jj[pk] + 1.0), RES, RESh);
 }
 
-__global__ __launch_bounds__(256) void k_comm121(DevBasis B, const OneTask* tasks, const double* L, int Lh,
+// 512 threads here and in k_comm221: a thread's items run one after the other,
+// each a chain of dependent reads (111, 121 and 221 with 256 / 512 threads: eMax
+// 6 28.0 / 24.0 us, 8 45.4 / 33.1, 10 71.7 / 54.3).
+__global__ __launch_bounds__(512) void k_comm121(DevBasis B, const OneTask* tasks, const double* L, int Lh,
                                                  const double* R, int Rh, double* RES, int RESh) {
-  __shared__ double red[256];
+  __shared__ double red[512];
   d_comm121(B, tasks, L, Lh, R, Rh, RES, RESh, blockIdx.x, red);
 }
 
 void launch_comm121(const DevBasis& B, const OneTask* t, int nt, const double* L, int Lh, const double* R,
                     int Rh, double* RES, int RESh, hipStream_t s) {
   if (nt <= 0) return;
-  hipLaunchKernelGGL(k_comm121, dim3(nt, B.ninst), dim3(256), 0, s, B, t, L, Lh, R, Rh, RES, RESh);
+  hipLaunchKernelGGL(k_comm121, dim3(nt, B.ninst), dim3(512), 0, s, B, t, L, Lh, R, Rh, RES, RESh);
 }
 
 // ============================================================ commutator_221
@@ -1121,17 +1124,17 @@ __device__ __forceinline__ void d_comm221(DevBasis B, const OneTask* tasks, cons
   if (threadIdx.x == 0) onebody_update(B, t, sm / (ji + 1.0), RES, RESh);
 }
 
-__global__ __launch_bounds__(256) void k_comm221(DevBasis B, const OneTask* tasks, const double* L, int Lh,
+__global__ __launch_bounds__(512) void k_comm221(DevBasis B, const OneTask* tasks, const double* L, int Lh,
                                                  const double* R, int Rh, const double* w1, const double* w2,
                                                  double* RES, int RESh) {
-  __shared__ double red[256];
+  __shared__ double red[512];
   d_comm221(B, tasks, L, Lh, R, Rh, w1, w2, RES, RESh, blockIdx.x, red);
 }
 
 void launch_comm221(const DevBasis& B, const OneTask* t, int nt, const double* L, int Lh, const double* R, int Rh,
                     const double* w1, const double* w2, double* RES, int RESh, hipStream_t s) {
   if (nt <= 0) return;
-  hipLaunchKernelGGL(k_comm221, dim3(nt, B.ninst), dim3(256), 0, s, B, t, L, Lh, R, Rh, w1, w2, RES, RESh);
+  hipLaunchKernelGGL(k_comm221, dim3(nt, B.ninst), dim3(512), 0, s, B, t, L, Lh, R, Rh, w1, w2, RES, RESh);
 }
 
 // ================================================= commutator_110 + 220 (E0)
@@ -1228,17 +1231,15 @@ void launch_e0_final_b(const DevBasis& B, const double* part, int use220, int us
 // commutators.f90:611-668.  The grouped GEMM leaves C = W1 - W2 =
 // L1 R1 - Rh L3 R3^T in w1's pppp block; RES1 += C - pm C^T.  Tile pair
 // (I,J), I <= J, of 64 x 64: both C tiles are staged through LDS so every
-// global access is a contiguous column run.  With ref_outputs the
-// reference's W1 and W2 are left in w1 / w2 (W2 formed here, rank nh).
-__device__ __forceinline__ double w2pp(const double* L3, const double* R3, int np, int nh, int Rh, int x, int y) {
-  double s = 0.0;
-  for (int h = 0; h < nh; ++h) s += L3[x + (i64)h * np] * R3[y + (i64)h * np];
-  return s * Rh;
-}
-
-__global__ __launch_bounds__(256) void k_pppp_sym(DevBasis B, const PairTask* tasks, const double* L, int Lh,
-                                                  const double* R, int Rh, double* RES, double* w1, double* w2,
-                                                  int ref_outputs) {
+// global access is a contiguous column run.  The reference's W1 and W2 are
+// left in w1 / w2 (W2 formed here, rank nh).
+// Bound by latency at small sizes: a thread of one of two halves (tile (I, J)
+// and tile (J, I)) issues the 16 loads of its elements and of RES at once, and
+// W2's columns of R3 are uniform to a wave (one row of L3 a lane).  With a
+// load, a test and a W2 sum per element, one after the other, 222_pp_hh took
+// 315 us at eMax 8, now 261.
+__global__ __launch_bounds__(512) void k_pppp_sym(DevBasis B, const PairTask* tasks, const double* L, int Lh,
+                                                  const double* R, int Rh, double* RES, double* w1, double* w2) {
   int inst;
   if (!batch_inst(B, inst)) return;
   L += (i64)inst * B.oplen;
@@ -1246,8 +1247,7 @@ __global__ __launch_bounds__(256) void k_pppp_sym(DevBasis B, const PairTask* ta
   RES += (i64)inst * B.oplen;
   w1 += (i64)inst * B.oplen;
   w2 += (i64)inst * B.oplen;
-  __shared__ double T1[64][65];   // C(I0 + x, J0 + y)
-  __shared__ double T2[64][65];   // C(J0 + x, I0 + y)
+  __shared__ double S[2][64][65];   // S[half][x][y] = C(X0 + x, Y0 + y) of the half's tile
   const PairTask t = tasks[blockIdx.x];
   const int q = t.q;
   const int np = B.dims[q * 3], nh = B.dims[q * 3 + 2];
@@ -1257,41 +1257,42 @@ __global__ __launch_bounds__(256) void k_pppp_sym(DevBasis B, const PairTask* ta
   double* X1 = RES + o1;
   double* W21 = w2 + o1;
   const int pm = Lh * Rh;
-  const int I0 = t.ti * 64, J0 = t.tj * 64;
-  const bool diag = (t.ti == t.tj);
-  for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-    const int x = e & 63, y = e >> 6;
-    T1[x][y] = (I0 + x < np && J0 + y < np) ? Cm[(I0 + x) + (i64)(J0 + y) * np] : 0.0;
-    if (!diag) T2[x][y] = (J0 + x < np && I0 + y < np) ? Cm[(J0 + x) + (i64)(I0 + y) * np] : 0.0;
+  const bool diag = t.ti == t.tj;
+  const int half = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  const int x = threadIdx.x & 63, y0 = 16 * (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3);
+  const int X0 = (half ? t.tj : t.ti) * 64, Y0 = (half ? t.ti : t.tj) * 64;
+  const int gx = X0 + x, cx = min(gx, np - 1);
+  double c[16], u[16];
+  if (!(diag && half)) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const i64 o = cx + (i64)min(Y0 + y0 + r, np - 1) * np;
+      c[r] = Cm[o];
+      u[r] = X1[o];
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) S[half][x][y0 + r] = c[r];
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-    const int x = e & 63, y = e >> 6;
-    const int gx = I0 + x, gy = J0 + y;
+  if (diag && half) return;
+  double w[16];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) w[r] = 0.0;
+  for (int h = 0; h < nh; ++h) {
+    const double l = L3[cx + (i64)h * np];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) w[r] += l * R3[min(Y0 + y0 + r, np - 1) + (i64)h * np];
+  }
+  const double (*St)[65] = S[diag ? 0 : 1 - half];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int gy = Y0 + y0 + r;
     if (gx < np && gy < np) {
-      const double cxy = T1[x][y];
-      const double cyx = diag ? T1[y][x] : T2[y][x];
       const i64 o = gx + (i64)gy * np;
-      X1[o] = X1[o] + cxy - cyx * pm;
-      if (ref_outputs) {
-        const double w2v = w2pp(L3, R3, np, nh, Rh, gx, gy);
-        Cm[o] = cxy + w2v;
-        W21[o] = w2v;
-      }
-    }
-    if (!diag) {
-      const int hx = J0 + x, hy = I0 + y;   // element (J0 + x, I0 + y) of tile (J, I)
-      if (hx < np && hy < np) {
-        const double cxy = T2[x][y];
-        const double cyx = T1[y][x];
-        const i64 o = hx + (i64)hy * np;
-        X1[o] = X1[o] + cxy - cyx * pm;
-        if (ref_outputs) {
-          const double w2v = w2pp(L3, R3, np, nh, Rh, hx, hy);
-          Cm[o] = cxy + w2v;
-          W21[o] = w2v;
-        }
-      }
+      const double w2v = w[r] * Rh;
+      X1[o] = u[r] + c[r] - St[y0 + r][x] * pm;
+      Cm[o] = c[r] + w2v;
+      W21[o] = w2v;
     }
   }
 }
@@ -1300,7 +1301,8 @@ __global__ __launch_bounds__(256) void k_pppp_sym(DevBasis B, const PairTask* ta
 // workgroup per output tile (two per off-diagonal pair, blockIdx.x = 2 task
 // + side), its own C tile read straight from memory and only the tile whose
 // transpose it needs staged in LDS (33 KB instead of 66 KB: twice the
-// workgroups per CU).  Same arithmetic as k_pppp_sym.
+// workgroups per CU).  Same arithmetic as k_pppp_sym.  A load and a test
+// at a time it took 14.2 us (eMax 6), 30.7 (8), 125 (10); now 6.4, 22.4, 112.
 __device__ __forceinline__ void d_pppp_sym1(DevBasis B, const PairTask* tasks, double* RES, const double* w1,
                                             int pm, int upper_only, int bx, double (*S)[65]) {
   int inst;
@@ -1321,20 +1323,24 @@ __device__ __forceinline__ void d_pppp_sym1(DevBasis B, const PairTask* tasks, d
   double* X1 = RES + o1;
   // output tile rows R0.., cols C0..; source tile rows C0.., cols R0..
   const int R0 = (side == 0 ? t.ti : t.tj) * 64, C0 = (side == 0 ? t.tj : t.ti) * 64;
-  for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-    const int x = e & 63, y = e >> 6;
-    S[x][y] = (C0 + x < np && R0 + y < np) ? Cm[(C0 + x) + (i64)(R0 + y) * np] : 0.0;
+  // every load of a thread before the barrier, at valid addresses
+  const int x = threadIdx.x & 63, y0 = threadIdx.x >> 6;
+  double c[16], u[16], v[16];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int y = y0 + 4 * r;
+    const i64 o = min(R0 + x, np - 1) + (i64)min(C0 + y, np - 1) * np;
+    v[r] = Cm[min(C0 + x, np - 1) + (i64)min(R0 + y, np - 1) * np];
+    c[r] = Cm[o];
+    u[r] = X1[o];
   }
+#pragma unroll
+  for (int r = 0; r < 16; ++r) S[x][y0 + 4 * r] = v[r];
   __syncthreads();
-  for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-    const int x = e & 63, y = e >> 6;
-    const int gx = R0 + x, gy = C0 + y;
-    if (gx < np && gy < np) {
-      const i64 o = gx + (i64)gy * np;
-      const double cxy = Cm[o];
-      const double cyx = S[y][x];
-      X1[o] = X1[o] + cxy - cyx * pm;
-    }
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int y = y0 + 4 * r, gx = R0 + x, gy = C0 + y;
+    if (gx < np && gy < np) X1[gx + (i64)gy * np] = u[r] + c[r] - S[y][x] * pm;
   }
 }
 
@@ -1353,7 +1359,7 @@ void launch_pppp_sym(const DevBasis& B, const PairTask* t, int nt, const double*
                        (const double*)w1, Lh * Rh, upper_only);
     return;
   }
-  hipLaunchKernelGGL(k_pppp_sym, dim3(nt, B.ninst), dim3(256), 0, s, B, t, L, Lh, R, Rh, RES, w1, w2, ref_outputs);
+  hipLaunchKernelGGL(k_pppp_sym, dim3(nt, B.ninst), dim3(512), 0, s, B, t, L, Lh, R, Rh, RES, w1, w2);
 }
 
 // ================================ 222_pp_hh epilogue of the small blocks
