@@ -1762,6 +1762,14 @@ int read_scalar(imsrg_basis_s* B, const double* dev, double* out, hipStream_t s)
   return 0;
 }
 
+// the norm that the last kernel of a nested commutator wrote to pinned host
+// memory (a copy of the device scalar instead cost a launch of its own)
+int read_norm(imsrg_basis_s* B, double* out, hipStream_t s) {
+  HIPCHK(hipStreamSynchronize(s));
+  *out = B->hval[0];
+  return 0;
+}
+
 // BCH_EXPAND, IMSRG_MAGNUS.f90:149-234
 int bch(imsrg_flow_s* F, double* HS, const double* G, int Gh, const double* H, int Hh, double conv, int maxit,
         int* nterms, double* advals, hipStream_t s, TermRec* rec = nullptr, size_t* pidx = nullptr) {
@@ -1784,7 +1792,7 @@ int bch(imsrg_flow_s* F, double* HS, const double* G, int Gh, const double* H, i
     const double c = coef;
     imsrg_flow_s::GraphKey key{0, iw, HS, G, H, Gh, Hh};
     int rc = run_term(F, key, s, [&](hipStream_t cs) {
-      const Append ap{HS, c, B->dval};
+      const Append ap{HS, c, B->hval};
       t_full(F->X, G, Gh, AD, Hh, INT2, Hh, true, F->w1, F->w2, F->GCC, F->ADCC, F->WCC, cs, &ap);
     });
     if (rc) return rc;
@@ -1796,7 +1804,7 @@ int bch(imsrg_flow_s* F, double* HS, const double* G, int Gh, const double* H, i
       rec->c.push_back(coef);
     }
     double nrm = 0.0;
-    if ((rc = read_scalar(B, B->dval, &nrm, s))) return rc;
+    if ((rc = read_norm(B, &nrm, s))) return rc;
     const double adv = nrm * coef;
     if (advals) advals[iw - 2] = adv;
     if (adv < conv) break;
@@ -1817,9 +1825,8 @@ int magnus(imsrg_flow_s* F, double* DG, int DGh, const double* G, int Gh, double
   // INT2 = DG (both ping-pong buffers carry DG's E0, which no term writes)
   HIPCHK(hipMemcpyAsync(F->buf[0], DG, n * sizeof(double), hipMemcpyDeviceToDevice, s));
   HIPCHK(hipMemcpyAsync(F->buf[1], DG, sizeof(double), hipMemcpyDeviceToDevice, s));
-  t_norm(F->X, DG, B->dval, s);
-  t_norm(F->X, G, B->dval + 1, s);
-  HIPCHK(hipMemcpyAsync(B->hval, B->dval, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
+  t_norm(F->X, DG, B->hval, s);
+  t_norm(F->X, G, B->hval + 1, s);
   HIPCHK(hipStreamSynchronize(s));
   advals[0] = B->hval[0];
   const double fullnorm = B->hval[1];
@@ -1840,7 +1847,7 @@ int magnus(imsrg_flow_s* F, double* DG, int DGh, const double* G, int Gh, double
     const double c = cof[i - 1];
     imsrg_flow_s::GraphKey key{1, i, DG, G, nullptr, Gh, DGh};
     rc = run_term(F, key, s, [&](hipStream_t cs) {
-      const Append ap{DG, c, B->dval};
+      const Append ap{DG, c, B->hval};
       t_full(F->X, G, Gh, AD, DGh, INT2, DGh, false, F->w1, F->w2, F->GCC, F->ADCC, F->WCC, cs, &ap);
     });
     if (rc) return rc;
@@ -1853,7 +1860,7 @@ int magnus(imsrg_flow_s* F, double* DG, int DGh, const double* G, int Gh, double
       rec->c.push_back(c);
     }
     double nrm = 0.0;
-    if ((rc = read_scalar(B, B->dval, &nrm, s))) return rc;
+    if ((rc = read_norm(B, &nrm, s))) return rc;
     advals[i - 1] = nrm * std::fabs(cof[i - 1]);
   }
   if (ncomm) *ncomm = cnt;
@@ -1919,9 +1926,8 @@ int magnus_step(imsrg_flow_s* F, double* HS, double* G, double* DG, const double
   launch_axpy(B->b.oplen, G, 1.0, DG, ds, G, s);   // euler_step
   if ((rc = bch(F, HS, G, -1, H, 1, bch_conv, 40, &nb, nullptr, s))) return rc;
   if ((rc = generator(F, F->X, HS, DG, s))) return rc;
-  if ((rc = mbpt2_dev(F->X, HS, B->dval + 2, s))) return rc;
-  HIPCHK(hipMemcpyAsync(B->dval + 3, HS, sizeof(double), hipMemcpyDeviceToDevice, s));
-  HIPCHK(hipMemcpyAsync(B->hval, B->dval + 2, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
+  if ((rc = mbpt2_dev(F->X, HS, B->hval, s))) return rc;
+  HIPCHK(hipMemcpyAsync(B->hval + 1, HS, sizeof(double), hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
   if (out) {
     out[0] = B->hval[1];
@@ -2112,11 +2118,11 @@ int bch_record(imsrg_flow_s* F, const double* G, const double* H, int Hh, double
     coef = coef / (iw - 1.0);
     double* nx = nullptr;
     if ((rc = pool_get(F, pidx, &nx))) return rc;
-    const Append ap{HS, coef, B->dval};
+    const Append ap{HS, coef, B->hval};
     t_full(F->X, G, -1, rec.A.back(), Hh, nx, Hh, true, F->w1, F->w2, F->GCC, F->ADCC, F->WCC, s, HS ? &ap : nullptr);
-    if (!HS) t_norm(F->X, nx, B->dval, s);
+    if (!HS) t_norm(F->X, nx, B->hval, s);
     double nrm = 0.0;
-    if ((rc = read_scalar(B, B->dval, &nrm, s))) return rc;
+    if ((rc = read_norm(B, &nrm, s))) return rc;
     rec.A.push_back(nx);
     rec.c.push_back(coef);
     if (nrm * coef < conv) break;
@@ -2163,9 +2169,8 @@ int magnus_record(imsrg_flow_s* F, const double* ETA, double* DG, const double* 
   rec.A.assign(1, ETA);
   rec.c.assign(1, 1.0);
   if (DG != ETA) HIPCHK(hipMemcpyAsync(DG, ETA, n * sizeof(double), hipMemcpyDeviceToDevice, s));
-  t_norm(F->X, ETA, B->dval, s);
-  t_norm(F->X, G, B->dval + 1, s);
-  HIPCHK(hipMemcpyAsync(B->hval, B->dval, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
+  t_norm(F->X, ETA, B->hval, s);
+  t_norm(F->X, G, B->hval + 1, s);
   HIPCHK(hipStreamSynchronize(s));
   advals[0] = B->hval[0];
   const double fullnorm = B->hval[1];
@@ -2180,10 +2185,10 @@ int magnus_record(imsrg_flow_s* F, const double* ETA, double* DG, const double* 
     double* nx = nullptr;
     if ((rc = pool_get(F, pidx, &nx))) return rc;
     HIPCHK(hipMemcpyAsync(nx, rec.A.back(), sizeof(double), hipMemcpyDeviceToDevice, s));
-    const Append ap{DG, cof[i - 1], B->dval};
+    const Append ap{DG, cof[i - 1], B->hval};
     t_full(F->X, G, -1, rec.A.back(), -1, nx, -1, false, F->w1, F->w2, F->GCC, F->ADCC, F->WCC, s, &ap);
     double nrm = 0.0;
-    if ((rc = read_scalar(B, B->dval, &nrm, s))) return rc;
+    if ((rc = read_norm(B, &nrm, s))) return rc;
     advals[i - 1] = nrm * std::fabs(cof[i - 1]);
     rec.A.push_back(nx);
     rec.c.push_back(cof[i - 1]);
