@@ -1231,6 +1231,57 @@ void t_tail(const Exec& X, double* RES, int RESh, const Append* ap, hipStream_t 
   launch_sum_sqrt_b(X.D, X.part, B->tail.n, ap->norm, kDStride, 1, s);
 }
 
+// The small bases whose commutator runs in three launches: every family on
+// 32 x 32 LDS tiles with its usual transposes, 122 by lists, 222_ph by chunks
+bool small_phases(const Exec& X) {
+  imsrg_basis_s* B = X.B;
+  auto fits = [](const GemmFamily& f, int sig) { return f.tasks.n == 0 || (f.tile == 5 && f.sig == sig); };
+  return B->path == IMSRG_PATH_GROUPED && !B->t122_ok && !B->phb_ok && fits(B->pp1, 8) && fits(B->k2, 0) &&
+         fits(B->k3, 1) && fits(B->ph, 10);
+}
+PhaseGemm phase_gemm(const Exec& X, const GemmFamily& f, const double* a, const double* b, const double* c, i64 st,
+                     i64 sc, double as = 1.0, double s2 = 1.0) {
+  PhaseGemm g{};
+  g.sl.p[0] = a; g.sl.p[1] = b; g.sl.p[2] = c;
+  g.sl.st[0] = st; g.sl.st[1] = st; g.sl.st[2] = sc;
+  g.sl.act = X.D.act;
+  g.probs = f.probs; g.tasks = f.tasks.dev; g.xm = f.tasks.xmap; g.n = f.tasks.n; g.grid = f.tasks.n ? f.tasks.grid : 0;
+  g.as = as; g.s2 = s2;
+  return g;
+}
+bool t_phases(const Exec& X, const double* L, int Lh, const double* R, int Rh, double* RES, int RESh, bool e0,
+              double* w1, double* w2, const double* LCC, double* RCC, double* WCC, hipStream_t s) {
+  imsrg_basis_s* B = X.B;
+  const i64 op = B->b.oplen;
+  Phase1 p{};
+  p.k2 = phase_gemm(X, B->k2, L, R, X.K2scr, op, X.D.sk2scr);
+  p.pp1 = phase_gemm(X, B->pp1, L, R, w1, op, op, 1.0, -(double)Rh);
+  p.k3 = phase_gemm(X, B->k3, L, R, X.Pscr, op, X.D.spscr);
+  p.seg = B->seg_tri.dev; p.n122 = B->seg_tri.n;
+  p.part = B->partners; p.partT = B->partT; p.pstride = B->pstride;
+  p.rowp = B->rowp; p.colp = B->colp; p.f1off = B->f1off; p.nf1 = B->nf1;
+  p.cc = B->cc.dev; p.ncc = B->cc.n;
+  p.L = L; p.R = R; p.Lh = Lh; p.Rh = Rh; p.RES = RES; p.RESh = RESh;
+  p.RCC = RCC; p.epart = X.part;
+  if (!launch_phase1(X.D, p, e0, s)) return false;
+  Phase2 q{};
+  q.ph = phase_gemm(X, B->ph, LCC, RCC, WCC, B->b.cclen, B->b.wclen, (double)Lh, -(double)(Rh * Lh));
+  q.pairs = B->pairs.dev; q.npairs = B->pairs.n;
+  q.epi = B->seg_epi.dev; q.nepi = B->seg_epi.n;
+  q.L = L; q.R = R; q.Lh = Lh; q.Rh = Rh; q.RES = RES; q.w1 = w1; q.w2 = w2;
+  q.Pscr = X.Pscr; q.poff = B->poff; q.k3ks = B->k3ks; q.K2scr = X.K2scr; q.k2off = B->k2off; q.k2ks = B->k2ks;
+  q.epart = X.part;
+  launch_phase2(X.D, q, e0, s);
+  Phase3 r{};
+  r.one = B->one; r.none = (int)B->one_h.size();
+  r.phc = B->phc; r.nphc = (int)B->phc_h.size();
+  r.fq = B->fq; r.fql = B->fql; r.fqi = B->fqi; r.quad = B->quad;
+  r.L = L; r.R = R; r.Lh = Lh; r.Rh = Rh; r.RES = RES; r.RESh = RESh;
+  r.w1 = w1; r.w2 = w2; r.WCC = WCC;
+  launch_phase3(X.D, r, s);
+  return true;
+}
+
 // RES = [L, R]: the term sequence of BCH_EXPAND / MAGNUS_EXPAND
 // (IMSRG_MAGNUS.f90:207-219, 677-683).  LCC must already hold the
 // cross-coupled L (t_cc); RCC is computed here.
@@ -1243,6 +1294,10 @@ void t_full(const Exec& X, const double* L, int Lh, const double* R, int Rh, dou
   // accumulated on the way)
   const bool mirror = X.B->path != IMSRG_PATH_GROUPED;
   imsrg_basis_s* B = X.B;
+  if (small_phases(X) && t_phases(X, L, Lh, R, Rh, RES, RESh, e0, w1, w2, LCC, RCC, WCC, s)) {
+    t_tail(X, RES, RESh, ap, s);
+    return;
+  }
   if (!mirror && B->term_streams && B->aux_ready) {
     // Concurrent schedule, same results: RES's two-body part is still
     // written in the reference order (122, pppp, the other 222_pp_hh

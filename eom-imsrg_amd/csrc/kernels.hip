@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 
 #include "device.hpp"
+#include "gemm_tile.hpp"
 #include "kernels.hpp"
 
 namespace imsrg {
@@ -1972,6 +1973,110 @@ void launch_hf_unpack(const DevBasis& B, const SegTask* t, int nt, const double*
                       hipStream_t s) {
   if (nt <= 0) return;
   hipLaunchKernelGGL(k_hf_unpack, dim3(nt), dim3(kTile), 0, s, B, t, V, voff, op);
+}
+
+// ==================================== a small commutator in three launches
+// At eMax <= 4 every term kernel of the fused commutator lasts 4 - 13 us, a
+// few dependent memory latencies, and a graph of fourteen of them with joins
+// between queues spends as long between kernels as in them.  Here the terms
+// that do not wait for each other share a launch, one range of workgroups
+// each, the longest first: the bodies, and so the sums, are those of the
+// separate kernels.  Decoupling eMax 4 (174 nested commutators) 20.5 -> 10.6 ms.
+// Larger bases fill the chip term by term and take kernels that do not fit
+// here (register-direct tiles, block quadruples).
+union PhaseLds {
+  GemmLds<32, 32> g;
+  double s[64][65];
+  double f[64 * 65];
+};
+
+template <int SIG>
+__device__ __forceinline__ void phase_gemm(PhaseLds& lds, const PhaseGemm& f, int bx) {
+  const int ti = xcd_task(f.xm, bx);
+  if (ti < 0 || ti >= f.n) return;   // the range is rounded up
+  gemm_tile<32, 32, SIG>(lds.g, f.sl, f.probs, f.tasks[ti], blockIdx.y, f.as, f.s2);
+}
+
+__global__ __launch_bounds__(256) void k_phase1(DevBasis B, Phase1 P) {
+  __shared__ PhaseLds lds;
+  int inst;
+  if (!batch_inst(B, inst)) return;
+  int b = blockIdx.x;
+  if (b < P.k2.grid) return phase_gemm<0>(lds, P.k2, b);
+  b -= P.k2.grid;
+  if (b < P.pp1.grid) return phase_gemm<8>(lds, P.pp1, b);
+  b -= P.pp1.grid;
+  if (b < P.k3.grid) return phase_gemm<1>(lds, P.k3, b);
+  b -= P.k3.grid;
+  if (b < P.g122) {
+    if (b < P.n122)
+      d_comm122p(B, P.seg, P.part, P.partT, P.pstride, P.rowp, P.colp, P.f1off, P.nf1, P.L, P.Lh, P.R, P.Rh, P.RES,
+                 P.RESh, 0, b, P.n122, lds.f);
+    return;
+  }
+  b -= P.g122;
+  if (b < P.gcc) {
+    if (b < P.ncc) d_pandya(B, P.cc, P.R, P.Rh, P.RCC, b, P.ncc);
+    return;
+  }
+  b -= P.gcc;
+  if (b < P.n111) return d_comm111(B, P.L, P.Lh, P.R, P.Rh, P.RES, b);
+  b -= P.n111;
+  d_e0_partials(B, P.L, P.Lh, P.R, P.Rh, P.epart, b, lds.f);
+}
+
+__global__ __launch_bounds__(256) void k_phase2(DevBasis B, Phase2 P) {
+  __shared__ PhaseLds lds;
+  int inst;
+  if (!batch_inst(B, inst)) return;
+  int b = blockIdx.x;
+  if (b < P.ph.grid) return phase_gemm<10>(lds, P.ph, b);
+  b -= P.ph.grid;
+  if (b < P.npairs) return d_pppp_sym1(B, P.pairs, P.RES, P.w1, P.Lh * P.Rh, 1, b, lds.s);
+  b -= P.npairs;
+  if (b < P.nepi)
+    return d_pphh_epilogue(B, P.epi, P.L, P.Lh, P.R, P.Rh, P.RES, P.w1, P.w2, P.Pscr, P.poff, P.k3ks, P.K2scr,
+                           P.k2off, P.k2ks, b);
+  d_e0_final(P.epart, B.nblocks, P.Lh * P.Rh == -1 ? 1 : 0, 1, P.RES, 0, B.spart, B.oplen, B.act, lds.f);
+}
+
+// 121 and 221 of a one-body element in its workgroup, in that order
+__global__ __launch_bounds__(512) void k_phase3(DevBasis B, Phase3 P) {
+  __shared__ union { PhChunkLds c; double red[512]; } lds;
+  int inst;
+  if (!batch_inst(B, inst)) return;
+  int b = blockIdx.x;
+  if (b < P.g1) {
+    if (b >= P.none) return;
+    d_comm121(B, P.one, P.L, P.Lh, P.R, P.Rh, P.RES, P.RESh, b, lds.red);
+    __syncthreads();
+    d_comm221(B, P.one, P.L, P.Lh, P.R, P.Rh, P.w1, P.w2, P.RES, P.RESh, b, lds.red);
+    return;
+  }
+  b -= P.g1;
+  d_comm222ph_chunk(B, P.phc, P.fq, P.fql, P.fqi, P.quad, P.WCC, P.Lh, P.Rh, P.RES, P.RESh, 0, b, P.nphc, lds.c);
+}
+
+bool launch_phase1(const DevBasis& B, Phase1 P, int e0, hipStream_t s) {
+  if (2 * P.nf1 * sizeof(double) > sizeof(PhaseLds)) return false;
+  const i64 n = (i64)B.A * B.A + (i64)B.P * B.A + (i64)B.P * B.P;
+  auto up = [](int x) { return (x + kXcds - 1) / kXcds * kXcds; };   // ranges start on XCD 0, as the task orders assume
+  P.k2.grid = up(P.k2.grid); P.pp1.grid = up(P.pp1.grid); P.k3.grid = up(P.k3.grid);
+  P.g122 = up(P.n122); P.gcc = up(P.ncc);
+  P.n111 = (int)((n + 3) / 4);
+  const int grid = P.k2.grid + P.pp1.grid + P.k3.grid + P.g122 + P.gcc + P.n111 + (e0 ? B.nblocks + 1 : 0);
+  if (grid > 0) hipLaunchKernelGGL(k_phase1, dim3(grid, B.ninst), dim3(256), 0, s, B, P);
+  return true;
+}
+void launch_phase2(const DevBasis& B, Phase2 P, int e0, hipStream_t s) {
+  P.ph.grid = (P.ph.grid + kXcds - 1) / kXcds * kXcds;
+  const int grid = P.ph.grid + P.npairs + P.nepi + (e0 ? 1 : 0);
+  if (grid > 0) hipLaunchKernelGGL(k_phase2, dim3(grid, B.ninst), dim3(256), 0, s, B, P);
+}
+void launch_phase3(const DevBasis& B, Phase3 P, hipStream_t s) {
+  P.g1 = (P.none + kXcds - 1) / kXcds * kXcds;
+  const int grid = P.g1 + P.nphc;
+  if (grid > 0) hipLaunchKernelGGL(k_phase3, dim3(grid, B.ninst), dim3(512), 0, s, B, P);
 }
 
 }  // namespace imsrg

@@ -306,4 +306,39 @@ void launch_gen_vjp(const DevBasis& B, const SegTask* g3, int ng3, const double*
 void launch_normal_order_vjp(const DevBasis& B, const double* Hb, double* Tb, hipStream_t s);
 void launch_add_e0(double* dst, const double* src, double factor, hipStream_t s);
 
+// The fused commutator of a small basis in three launches (k_phase1, 2, 3)
+struct PhaseGemm { Slots sl; const GemmProb* probs; const GemmTask* tasks; XcdMap xm; int n, grid; double as, s2; };
+struct Phase1 {   // 222_pp_hh products, 122, Pandya of R, 111, E0 partial sums
+  PhaseGemm k2, pp1, k3;
+  const SegTask* seg; int n122, g122;
+  const Partner *part, *partT; int pstride;
+  const int *rowp, *colp, *f1off; int nf1;
+  const CCTask* cc; int ncc, gcc;
+  int n111;
+  const double *L, *R; int Lh, Rh;
+  double *RES; int RESh;
+  double *RCC, *epart;
+};
+struct Phase2 {   // W', the pppp and the other 222_pp_hh epilogues, E0
+  PhaseGemm ph;
+  const PairTask* pairs; int npairs;
+  const SegTask* epi; int nepi;
+  const double *L, *R; int Lh, Rh;
+  double *RES, *w1, *w2;
+  const double *Pscr; const i64* poff; const int* k3ks;
+  const double *K2scr; const i64* k2off; const int* k2ks;
+  double* epart;
+};
+struct Phase3 {   // 121 and 221, inverse Pandya
+  const OneTask* one; int none, g1;
+  const PhChunk* phc; int nphc;
+  const int *fq, *fql, *fqi; const QuadItem* quad;
+  const double *L, *R; int Lh, Rh;
+  double *RES; int RESh;
+  const double *w1, *w2, *WCC;
+};
+bool launch_phase1(const DevBasis& B, Phase1 P, int e0, hipStream_t s);   // false: the basis does not fit
+void launch_phase2(const DevBasis& B, Phase2 P, int e0, hipStream_t s);
+void launch_phase3(const DevBasis& B, Phase3 P, hipStream_t s);
+
 }  // namespace imsrg
