@@ -513,6 +513,80 @@ __global__ __launch_bounds__(64) void k_ts_ph(DevBasis B, DevTensor T, const TPh
   }
 }
 
+// Both terms for a small tensor, one thread per output element: a pack's wave
+// runs through all its terms one after the other, and a few hundred packs do
+// not fill the chip (launch_ts212 / launch_ts_ph have the figures).
+__global__ __launch_bounds__(256) void k_ts212_out(DevBasis B, DevTensor T, const TPh* tasks, i64 nt, const double* L,
+                                                   int Lh, const double* R, int Rh, double* RES) {
+  const i64 e = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= nt) return;
+  const TPh t = tasks[e];
+  const int rank = T.rank, nr = rank + 1, J1 = t.jj & 0xffff, J2 = t.jj >> 16;
+  const int a = t.abcd & 255, b = (t.abcd >> 8) & 255, c = (t.abcd >> 16) & 255, d = (t.abcd >> 24) & 255;
+  const int ja = B.jj[a], jb = B.jj[b], jc = B.jj[c], jd = B.jj[d];
+  double s1 = 0.0, s2 = 0.0, s3 = 0.0, s4 = 0.0;
+  for (int k = T.fst[a * nr]; k < T.fst[(a + 1) * nr]; ++k) {
+    const int i = T.fmem[k];
+    s1 = s1 - x6(T, J1, J2, B.jj[i], ja, jb) * f_tensor_elem(B, R, Rh, a, i) * v_elem(B, L, Lh, i, b, c, d, J2);
+  }
+  for (int k = T.fst[b * nr]; k < T.fst[(b + 1) * nr]; ++k) {
+    const int i = T.fmem[k];
+    s2 = s2 + x6(T, J1, J2, B.jj[i], jb, ja) * f_tensor_elem(B, R, Rh, b, i) * v_elem(B, L, Lh, i, a, c, d, J2);
+  }
+  for (int k = T.fst[d * nr]; k < T.fst[(d + 1) * nr]; ++k) {
+    const int i = T.fmem[k];
+    s3 = s3 + x6(T, J1, J2, jd, B.jj[i], jc) * f_tensor_elem(B, R, Rh, i, d) * v_elem(B, L, Lh, a, b, c, i, J1);
+  }
+  for (int k = T.fst[c * nr]; k < T.fst[(c + 1) * nr]; ++k) {
+    const int i = T.fmem[k];
+    s4 = s4 - x6(T, J1, J2, jc, B.jj[i], jd) * f_tensor_elem(B, R, Rh, i, c) * v_elem(B, L, Lh, a, b, d, i, J1);
+  }
+  const double sm = s1 * m1pow((ja + jb - J2) / 2) + s2 * m1pow((J1 + J2) / 2) + s3 * m1pow((jc + jd - J1) / 2) +
+                    s4 * m1pow((J2 + J1) / 2);
+  RES[t.off] += sm * sqrt((J1 + 1.0) * (J2 + 1.0) / (1.0 + (a == b)) / (1.0 + (c == d))) * m1pow(rank / 2);
+}
+
+__global__ __launch_bounds__(256) void k_ts_ph_out(DevBasis B, DevTensor T, const TPh* tasks, i64 nt, int Lh, int Rh,
+                                                   const double* Wx, const double* Wy, double* RES) {
+  const i64 e = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= nt) return;
+  const TPh t = tasks[e];
+  const int u = t.abcd, R = T.rank, nR = R / 2 + 1, J1 = t.jj & 0xffff, J2 = t.jj >> 16;
+  const bool eqb = (u & 255) == ((u >> 8) & 255), eqk = ((u >> 16) & 255) == ((u >> 24) & 255);
+  if ((eqb && ((J1 >> 1) & 1)) || (eqk && ((J2 >> 1) & 1))) return;
+  const double thr = (double)1e-6f;
+  double sm = 0.0;
+  for (int pat = 0; pat < 16; ++pat) {
+    if ((eqb && ((kPatBra >> pat) & 1)) || (eqk && ((kPatKet >> pat) & 1))) continue;
+    const TPat x = ts_pat(pat, u);
+    const int Tz = abs(B.tz[x.d] - B.tz[x.a]) >> 1, PAR = (B.ll[x.d] + B.ll[x.a]) & 1;
+    if ((abs(B.tz[x.c] - B.tz[x.b]) >> 1) != Tz) continue;
+    if (((B.ll[x.c] + B.ll[x.b]) & 1) != ((PAR + (T.dpar >> 1)) & 1)) continue;
+    const int ja = B.jj[x.a], jb = B.jj[x.b], jc = B.jj[x.c], jd = B.jj[x.d];
+    const double* W = pat < 8 ? Wx : Wy;
+    const bool t2 = pat & 1, sw12 = (pat < 8) ? t2 : !t2, use34 = (kPat34 >> pat) & 1;
+    const int u1 = sw12 ? jd : ja, u2 = sw12 ? ja : jd, u4 = t2 ? jc : jb, u5 = t2 ? jb : jc;
+    double sp = 0.0;
+    for (int J3 = abs(jd - ja); J3 <= jd + ja; J3 += 2) {
+      const int IX = B.rmap[((i64)x.d * B.N + x.a) * B.nJ + (J3 >> 1)];
+      const int J4lo = max(max(max(abs(J3 - R), J3), abs(jc - jb)), pat < 8 ? J3 : J3 + 2);
+      const int J4hi = min(min(J3 + R, jc + jb), 2 * B.JTM);
+      for (int J4 = J4lo; J4 <= J4hi; J4 += 2) {
+        const i64* wt = T.wtab + ((((J3 >> 1) * nR + ((J4 - J3) >> 1)) << 2) + 2 * Tz + PAR) * 2;
+        const double w = W[wt[0] + IX + B.rmap[((i64)x.c * B.N + x.b) * B.nJ + (J4 >> 1)] * wt[1]];
+        if (!(fabs(w) > thr)) continue;
+        const double v = n9(T, u1, u2, J3, u4, u5, J4, J1, J2) * w;
+        sp += (use34 && (((J3 + J4) >> 1) & 1)) ? -v : v;
+      }
+    }
+    sm += ts_pat_coef(pat, ja, jb, jc, jd, J1, J2, R, Lh, Rh) * sp;
+  }
+  sm *= sqrt((J1 + 1.0) * (J2 + 1.0));
+  if (eqb) sm *= 1.4142135623730951;
+  if (eqk) sm *= 1.4142135623730951;
+  RES[t.off] += sm;
+}
+
 // calculate_single_pandya, cross_coupled.f90:1416-1634, one thread per
 // element of CCX(qx) (term 1: r1 x nb2) or CCR(qx) (term 2: nb1 x r2)
 // J4 runs only where the tensor couples it to J3 (over its whole range, with a
@@ -625,14 +699,28 @@ void launch_ts122(const DevBasis& B, const DevTensor& T, const TSub* sb, const T
   if (nt > 0) hipLaunchKernelGGL(k_ts122, dim3(nt), dim3(256), 0, s, B, T, sb, t, L, Lh, R, Rh, RES);
 }
 
-void launch_ts212(const DevBasis& B, const DevTensor& T, const TPh* t, const TPack* p, int np, const int2* q,
+// From kTsPackMin outputs on by packs of quadruples.  Whole commutator, us, by
+// output / by packs: eMax 3 rank 4 (32 k outputs) 424 / 631, eMax 4 rank 4 (179 k)
+// 641 / 901, eMax 5 rank 2 (549 k) 867 / 929, rank 4 (754 k) 1331 / 1409, eMax 6
+// rank 2 odd parity (1.85 M) 2099 / 1628, rank 4 (2.6 M) 3623 / 2975.
+constexpr i64 kTsPackMin = 800000;
+void launch_ts212(const DevBasis& B, const DevTensor& T, const TPh* t, i64 nt, const TPack* p, int np, const int2* q,
                   const double* L, int Lh, const double* R, int Rh, double* RES, hipStream_t s) {
-  if (np > 0) hipLaunchKernelGGL(k_ts212, dim3(np), dim3(64), 0, s, B, T, t, p, q, L, Lh, R, Rh, RES);
+  if (nt <= 0) return;
+  if (nt < kTsPackMin)
+    hipLaunchKernelGGL(k_ts212_out, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, s, B, T, t, nt, L, Lh, R, Rh, RES);
+  else
+    hipLaunchKernelGGL(k_ts212, dim3(np), dim3(64), 0, s, B, T, t, p, q, L, Lh, R, Rh, RES);
 }
 
-void launch_ts_ph(const DevBasis& B, const DevTensor& T, const TPh* t, const TPack* p, int np, const int2* q, int Lh,
-                  int Rh, const double* Wx, const double* Wy, double* RES, hipStream_t s) {
-  if (np > 0) hipLaunchKernelGGL(k_ts_ph, dim3(np), dim3(64), 0, s, B, T, t, p, q, Lh, Rh, Wx, Wy, RES);
+void launch_ts_ph(const DevBasis& B, const DevTensor& T, const TPh* t, i64 nt, const TPack* p, int np, const int2* q,
+                  int Lh, int Rh, const double* Wx, const double* Wy, double* RES, hipStream_t s) {
+  if (nt <= 0) return;
+  if (nt < kTsPackMin)
+    hipLaunchKernelGGL(k_ts_ph_out, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, s, B, T, t, nt, Lh, Rh, Wx, Wy,
+                       RES);
+  else
+    hipLaunchKernelGGL(k_ts_ph, dim3(np), dim3(64), 0, s, B, T, t, p, q, Lh, Rh, Wx, Wy, RES);
 }
 void launch_ts_pandya(const DevBasis& B, const DevTensor& T, const TCC* t, int nt, const double* R, int Rh,
                       double* CC, hipStream_t s) {

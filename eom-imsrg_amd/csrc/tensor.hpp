@@ -99,11 +99,11 @@ void launch_ts_one(int mode, const DevBasis& B, const DevTensor& T, const TOne* 
 void launch_ts122(const DevBasis& B, const DevTensor& T, const TSub* sb, const TElem* t, int nt, const double* L,
                   int Lh, const double* R, int Rh, double* RES, hipStream_t s);
 // TS_commutator_212 (adds)
-void launch_ts212(const DevBasis& B, const DevTensor& T, const TPh* t, const TPack* p, int np, const int2* q,
+void launch_ts212(const DevBasis& B, const DevTensor& T, const TPh* t, i64 nt, const TPack* p, int np, const int2* q,
                   const double* L, int Lh, const double* R, int Rh, double* RES, hipStream_t s);
 // the back-transform of TS_commutator_222_ph from the products Wx / Wy
-void launch_ts_ph(const DevBasis& B, const DevTensor& T, const TPh* t, const TPack* p, int np, const int2* q, int Lh,
-                  int Rh, const double* Wx, const double* Wy, double* RES, hipStream_t s);
+void launch_ts_ph(const DevBasis& B, const DevTensor& T, const TPh* t, i64 nt, const TPack* p, int np, const int2* q,
+                  int Lh, int Rh, const double* Wx, const double* Wy, double* RES, hipStream_t s);
 // calculate_single_pandya of every listed (block, term) into CC
 void launch_ts_pandya(const DevBasis& B, const DevTensor& T, const TCC* t, int nt, const double* R, int Rh,
                       double* CC, hipStream_t s);
