@@ -515,7 +515,7 @@ __global__ __launch_bounds__(64) void k_ts_ph(DevBasis B, DevTensor T, const TPh
 
 // Both terms for a small tensor, one thread per output element: a pack's wave
 // runs through all its terms one after the other, and a few hundred packs do
-// not fill the chip (launch_ts212 / launch_ts_ph have the figures).
+// not fill the chip (kTsPackMin has the figures).
 __global__ __launch_bounds__(256) void k_ts212_out(DevBasis B, DevTensor T, const TPh* tasks, i64 nt, const double* L,
                                                    int Lh, const double* R, int Rh, double* RES) {
   const i64 e = (i64)blockIdx.x * blockDim.x + threadIdx.x;
@@ -699,15 +699,11 @@ void launch_ts122(const DevBasis& B, const DevTensor& T, const TSub* sb, const T
   if (nt > 0) hipLaunchKernelGGL(k_ts122, dim3(nt), dim3(256), 0, s, B, T, sb, t, L, Lh, R, Rh, RES);
 }
 
-// From kTsPackMin outputs on by packs of quadruples.  Whole commutator, us, by
-// output / by packs: eMax 3 rank 4 (32 k outputs) 424 / 631, eMax 4 rank 4 (179 k)
-// 641 / 901, eMax 5 rank 2 (549 k) 867 / 929, rank 4 (754 k) 1331 / 1409, eMax 6
-// rank 2 odd parity (1.85 M) 2099 / 1628, rank 4 (2.6 M) 3623 / 2975.
-constexpr i64 kTsPackMin = 800000;
+// by packs where the tensor has them (npacks > 0), else one thread per output
 void launch_ts212(const DevBasis& B, const DevTensor& T, const TPh* t, i64 nt, const TPack* p, int np, const int2* q,
                   const double* L, int Lh, const double* R, int Rh, double* RES, hipStream_t s) {
   if (nt <= 0) return;
-  if (nt < kTsPackMin)
+  if (np == 0)
     hipLaunchKernelGGL(k_ts212_out, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, s, B, T, t, nt, L, Lh, R, Rh, RES);
   else
     hipLaunchKernelGGL(k_ts212, dim3(np), dim3(64), 0, s, B, T, t, p, q, L, Lh, R, Rh, RES);
@@ -716,7 +712,7 @@ void launch_ts212(const DevBasis& B, const DevTensor& T, const TPh* t, i64 nt, c
 void launch_ts_ph(const DevBasis& B, const DevTensor& T, const TPh* t, i64 nt, const TPack* p, int np, const int2* q,
                   int Lh, int Rh, const double* Wx, const double* Wy, double* RES, hipStream_t s) {
   if (nt <= 0) return;
-  if (nt < kTsPackMin)
+  if (np == 0)
     hipLaunchKernelGGL(k_ts_ph_out, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, s, B, T, t, nt, Lh, Rh, Wx, Wy,
                        RES);
   else

@@ -56,6 +56,12 @@ struct TPh { int off, abcd, jj; };
 // at most 64 quadruples of that list (quads q0 .. q0 + nq: orbits, first
 // output) with the same four j, patterns and outputs (J1, J2)
 struct TPack { int q0, nq, no; unsigned mask; };
+// From kTsPackMin outputs on 212 and 222_ph run by packs of quadruples, below
+// one thread per output.  Whole commutator, us, by output / by packs: eMax 3 rank 4
+// (32 k outputs) 424 / 631, eMax 4 rank 4 (179 k) 641 / 901, eMax 5 rank 2 (549 k)
+// 867 / 929, rank 4 (754 k) 1331 / 1409, eMax 6 rank 2 odd parity (1.85 M) 2099 /
+// 1628, rank 4 (2.6 M) 3623 / 2975.
+constexpr i64 kTsPackMin = 800000;
 constexpr int kTsOut = 16;    // outputs a lane accumulates at a time
 constexpr int kTsRows = 64;   // (J3, J4) pairs whose coefficients are staged at a time
 

@@ -145,7 +145,7 @@ SIGNATURES = {
     "imsrg_tensor_frob_norm": (_i, [_p, _dp, _d, _p]),
     "imsrg_tensor_add": (_i, [_p, _dp, C.c_double, _dp, C.c_double, _dp, _p]),
 }
-TSIZE = dict(OP=0, NBLOCKS=1, NCC=2, CC=3, W=4)
+TSIZE = dict(OP=0, NBLOCKS=1, NCC=2, CC=3, W=4, PACKS=5)
 
 GEMM = dict(PPPP=0, PPX=1, XX=2, PH=3, ADJ=4, ADJ_PH=5, ADJ_PP=6)
 GENERATOR = dict(white=0, atan=1, w2=2)

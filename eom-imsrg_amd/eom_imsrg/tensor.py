@@ -42,6 +42,11 @@ class TensorLayout:
                                                 goff.ctypes.data_as(C.POINTER(C.c_int64))))
         self.info, self.dims, self.goff = info.reshape(nb, 7), dims.reshape(nb, 6), goff.reshape(nb, 9)
 
+    @property
+    def packs(self) -> int:
+        """waves of 212 and 222_ph by packs (0: one thread per output, or not used yet)"""
+        return int(_lib.lib.imsrg_tensor_size(self.handle, _lib.TSIZE["PACKS"]))
+
     SEA1 = (0, 0, 0, 1, 2, 1, 2, 1, 2)
     SEA2 = (0, 1, 2, 1, 2, 2, 0, 0, 1)
 

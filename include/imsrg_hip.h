@@ -448,6 +448,7 @@ int imsrg_profile_kernel(imsrg_basis b, int which, const double* L, int Lherm, c
 #define IMSRG_TSIZE_NCC 2     /* tensor cross-coupled blocks (pandya_mat) */
 #define IMSRG_TSIZE_CC 3      /* doubles of a tensor cross-coupled set: CCX and CCR of every block */
 #define IMSRG_TSIZE_W 4       /* doubles of one 222_ph product set (Wx or Wy of every block) */
+#define IMSRG_TSIZE_PACKS 5   /* waves of 212 and 222_ph by packs (0: one thread per output, or not used yet) */
 /* allocate_tensor + allocate_small_tensor_CCMAT + store_6j_3halfint
  * (basic_IMSRG.f90:688-951,2335-2411; cross_coupled.f90:498-700): rank and
  * dpar twice lambda and twice the parity change (STOP 'RANK MUST BE
