@@ -56,12 +56,15 @@ struct TPh { int off, abcd, jj; };
 // at most 64 quadruples of that list (quads q0 .. q0 + nq: orbits, first
 // output) with the same four j, patterns and outputs (J1, J2)
 struct TPack { int q0, nq, no; unsigned mask; };
-// From kTsPackMin outputs on 212 and 222_ph run by packs of quadruples, below
-// one thread per output.  Whole commutator, us, by output / by packs: eMax 3 rank 4
-// (32 k outputs) 424 / 631, eMax 4 rank 4 (179 k) 641 / 901, eMax 5 rank 2 (549 k)
-// 867 / 929, rank 4 (754 k) 1331 / 1409, eMax 6 rank 2 odd parity (1.85 M) 2099 /
-// 1628, rank 4 (2.6 M) 3623 / 2975.
-constexpr i64 kTsPackMin = 800000;
+// 212 and 222_ph run by packs from kTsPackMin orbit quadruples on, below by one
+// thread per output: a pack's wave runs through its terms one after the other,
+// so few packs (about nq / 50) leave the chip waiting, however many outputs a
+// quadruple has.  Whole commutator, us, by output / by packs: eMax 4 rank 8 (33 k
+// quadruples) 820 / 1565, eMax 5 rank 0 (122 k) 386 / 395, rank 4 (135 k) 1327 / 1404,
+// rank 8 (128 k, 888 k outputs) 1826 / 2411; eMax 14 lMax 1 rank 2 (180 k) 569 / 510,
+// eMax 6 rank 0 (376 k) 754 / 665, rank 4 (415 k) 3620 / 2971, eMax 7 lMax 5 rank 4
+// (727 k) 6428 / 3921.
+constexpr i64 kTsPackMin = 160000;
 constexpr int kTsOut = 16;    // outputs a lane accumulates at a time
 constexpr int kTsRows = 64;   // (J3, J4) pairs whose coefficients are staged at a time
 
