@@ -128,6 +128,7 @@ SIGNATURES = {
     "imsrg_tensor_create": (_i, [_p, _i, _i, C.POINTER(_p)]),
     "imsrg_tensor_destroy": (_i, [_p]),
     "imsrg_tensor_size": (C.c_int64, [_p, _i]),
+    "imsrg_tensor_set_form": (_i, [_p, _i]),
     "imsrg_tensor_blocks": (_i, [_p, _ip, _ip, _lp]),
     "imsrg_tensor_op_put": (_i, [_p, _dp, _i, _i, _d]),
     "imsrg_tensor_op_get": (_i, [_p, _dp, _i, _i, _d]),
@@ -146,6 +147,7 @@ SIGNATURES = {
     "imsrg_tensor_add": (_i, [_p, _dp, C.c_double, _dp, C.c_double, _dp, _p]),
 }
 TSIZE = dict(OP=0, NBLOCKS=1, NCC=2, CC=3, W=4, PACKS=5)
+TENSOR_FORM = dict(size=0, outputs=1, packs=2)
 
 GEMM = dict(PPPP=0, PPX=1, XX=2, PH=3, ADJ=4, ADJ_PH=5, ADJ_PP=6)
 GENERATOR = dict(white=0, atan=1, w2=2)

@@ -42,6 +42,10 @@ class TensorLayout:
                                                 goff.ctypes.data_as(C.POINTER(C.c_int64))))
         self.info, self.dims, self.goff = info.reshape(nb, 7), dims.reshape(nb, 6), goff.reshape(nb, 9)
 
+    def set_form(self, form: str) -> None:
+        """how 212 and 222_ph run ("size" picks, "outputs", "packs"); before the first use on the device"""
+        _lib.check(_lib.lib.imsrg_tensor_set_form(self.handle, _lib.TENSOR_FORM[form]))
+
     @property
     def packs(self) -> int:
         """waves of 212 and 222_ph by packs (0: one thread per output, or not used yet)"""

@@ -773,6 +773,12 @@ module imsrg_hip_c
       type(c_ptr), value :: t
       integer(c_int), value :: what
     end function imsrg_tensor_size
+    function imsrg_tensor_set_form(t, form) bind(C, name="imsrg_tensor_set_form")
+      import
+      integer(c_int) :: imsrg_tensor_set_form
+      type(c_ptr), value :: t
+      integer(c_int), value :: form
+    end function imsrg_tensor_set_form
     function imsrg_tensor_blocks(t, info, dims, goff) bind(C, name="imsrg_tensor_blocks")
       import
       integer(c_int) :: imsrg_tensor_blocks

@@ -457,6 +457,13 @@ int imsrg_profile_kernel(imsrg_basis b, int which, const double* L, int Lherm, c
 int imsrg_tensor_create(imsrg_basis b, int rank, int dpar, imsrg_tensor* out);
 int imsrg_tensor_destroy(imsrg_tensor t);
 int64_t imsrg_tensor_size(imsrg_tensor t, int what);
+/* How TS_commutator_212 and TS_commutator_222_ph run: one thread per output
+ * element or one wave per pack of alike orbit quadruples; by the tensor's size
+ * unless set here, before its first use on the device. */
+#define IMSRG_TENSOR_FORM_SIZE 0
+#define IMSRG_TENSOR_FORM_OUTPUTS 1
+#define IMSRG_TENSOR_FORM_PACKS 2
+int imsrg_tensor_set_form(imsrg_tensor t, int form);
 /* per block q: info[7q..] = 2J1, 2J2, Tz, P1, P2, channel of J1, channel of
  * J2 (-1: empty); dims[6q..] = npp1, nph1, nhh1, npp2, nph2, nhh2;
  * goff[9q..] offset of tgam g */

@@ -1,10 +1,10 @@
 """The two forms of the tensor terms 212 and 222_ph, one thread per output and
 one wave per pack of alike orbit quadruples: which one a tensor's size
-selects."""
+selects, and each against the oracle."""
 import pytest
 import torch
 
-from test_gpu_tensor import Basis, SqOp, tensor
+from test_gpu_tensor import Basis, CCMat, SqOp, _case, _close, cm, tensor
 
 pytestmark = pytest.mark.gpu
 
@@ -26,3 +26,42 @@ def _packs(emax, rank, dpar):
 def test_packs_only_where_they_run(emax, rank, dpar, by_packs):
     """a tensor whose terms run one thread per output holds no pack lists"""
     assert (_packs(emax, rank, dpar) > 0) == by_packs
+
+
+HERMS = [(-1, 1), (-1, -1), (1, 1), (1, -1)]
+
+
+@pytest.mark.parametrize("form", ["outputs", "packs"])
+@pytest.mark.parametrize("emax,rank,dpar", [(1, 2, 0), (2, 2, 2), (3, 8, 0), (3, 6, 2), (4, 4, 0)])
+def test_forms_vs_oracle(emax, rank, dpar, form):
+    """both forms of 212 and 222_ph against the oracle at every pair of
+    hermiticities: one shell, packs of one quadruple and of 64, more outputs than
+    a lane accumulates at a time, equal orbits in a pair, odd parity change"""
+    for hL, hR in HERMS:
+        b, o, ot, tl, L, R, P = _case(emax, rank, dpar, hL, hR, seed=7)
+        tl.set_form(form)
+        hC = -hL * hR
+        print(f"[tensor forms] eMax {emax} rank {rank} dpar {dpar} herm ({hL},{hR}) {form}", flush=True)
+        Ld, Rd = SqOp.from_numpy(b, L, hL), tensor.TensorOp.from_numpy(tl, R, hR)
+        LCC, RCC = CCMat(b, hL), tensor.TensorCC(tl)
+        cm.calculate_cross_coupled(Ld, LCC)
+        X = tensor.TensorOp.from_numpy(tl, P, hC)
+        tensor.TS_commutator_212(Ld, Rd, X)
+        _close(X.numpy(), ot.ts212(L, hL, R, hR, P.copy(), hC), f"212 {form} ({hL},{hR})")
+        X = tensor.TensorOp.from_numpy(tl, P, hC)
+        tensor.TS_commutator_222_ph(LCC, RCC, Rd, X)
+        _close(X.numpy(), ot.ts222ph(L, hL, R, hR, P.copy(), hC), f"222_ph {form} ({hL},{hR})")
+        assert (tl.packs > 0) == (form == "packs")
+
+
+def test_form_is_set_before_the_first_use():
+    from eom_imsrg import _lib
+    b = Basis.oxygen16(2)
+    tl = tensor.TensorLayout(b, 2, 0)
+    tl.set_form("packs")
+    tl.set_form("size")
+    with pytest.raises(_lib.ImsrgError):
+        _lib.check(_lib.lib.imsrg_tensor_set_form(tl.handle, 3))
+    tensor.TS_commutator_212(SqOp.zeros(b, -1), tensor.TensorOp.zeros(tl, 1), tensor.TensorOp.zeros(tl, 1))
+    with pytest.raises(_lib.ImsrgError):
+        tl.set_form("outputs")
