@@ -330,6 +330,34 @@ __global__ __launch_bounds__(256) void k_ts122(DevBasis B, DevTensor T, const TS
   RES[sb.off + IX + (i64)JX * sb.n1] = ts122(B, T, L, Lh, R, sb.q, IX, JX, a, b, c, d, J1, J2);
 }
 
+// TS_commutator_212 of one output element (TS_commutators.f90:666-806)
+__device__ __forceinline__ double ts212(const DevBasis& B, const DevTensor& T, const TPh& t, const double* L, int Lh,
+                                        const double* R, int Rh) {
+  const int rank = T.rank, nr = rank + 1, J1 = t.jj & 0xffff, J2 = t.jj >> 16;
+  const int a = t.abcd & 255, b = (t.abcd >> 8) & 255, c = (t.abcd >> 16) & 255, d = (t.abcd >> 24) & 255;
+  const int ja = B.jj[a], jb = B.jj[b], jc = B.jj[c], jd = B.jj[d];
+  double s1 = 0.0, s2 = 0.0, s3 = 0.0, s4 = 0.0;
+  for (int k = T.fst[a * nr]; k < T.fst[(a + 1) * nr]; ++k) {
+    const int i = T.fmem[k];
+    s1 = s1 - x6(T, J1, J2, B.jj[i], ja, jb) * f_tensor_elem(B, R, Rh, a, i) * v_elem(B, L, Lh, i, b, c, d, J2);
+  }
+  for (int k = T.fst[b * nr]; k < T.fst[(b + 1) * nr]; ++k) {
+    const int i = T.fmem[k];
+    s2 = s2 + x6(T, J1, J2, B.jj[i], jb, ja) * f_tensor_elem(B, R, Rh, b, i) * v_elem(B, L, Lh, i, a, c, d, J2);
+  }
+  for (int k = T.fst[d * nr]; k < T.fst[(d + 1) * nr]; ++k) {
+    const int i = T.fmem[k];
+    s3 = s3 + x6(T, J1, J2, jd, B.jj[i], jc) * f_tensor_elem(B, R, Rh, i, d) * v_elem(B, L, Lh, a, b, c, i, J1);
+  }
+  for (int k = T.fst[c * nr]; k < T.fst[(c + 1) * nr]; ++k) {
+    const int i = T.fmem[k];
+    s4 = s4 - x6(T, J1, J2, jc, B.jj[i], jd) * f_tensor_elem(B, R, Rh, i, c) * v_elem(B, L, Lh, a, b, d, i, J1);
+  }
+  const double sm = s1 * m1pow((ja + jb - J2) / 2) + s2 * m1pow((J1 + J2) / 2) + s3 * m1pow((jc + jd - J1) / 2) +
+                    s4 * m1pow((J2 + J1) / 2);
+  return sm * sqrt((J1 + 1.0) * (J2 + 1.0) / (1.0 + (a == b)) / (1.0 + (c == d))) * m1pow(rank / 2);
+}
+
 // TS_commutator_212 (TS_commutators.f90:666-806; adds), one wave per pack of
 // orbit quadruples that share their four j: of
 //   sum_i f(a i) v(i b c d; J2), f(b i) v(i a c d; J2),
@@ -339,6 +367,9 @@ __global__ __launch_bounds__(256) void k_ts122(DevBasis B, DevTensor T, const TS
 // partners of its orbit by their j.  The address unit (uncoalesced element
 // and pair-number reads) bounds it.  One thread per output, every orbit
 // tested: 10.5 -> 5.0 ms; over the partners only 9.7 (eMax 8, rank 4).
+// Every product meets every output, with a coefficient of zero at another J: an
+// infinite one would spread, so sums that are not finite are taken again by
+// output.
 __global__ __launch_bounds__(64) void k_ts212(DevBasis B, DevTensor T, const TPh* tasks, const TPack* packs,
                                               const int2* quads, const double* L, int Lh, const double* R, int Rh,
                                               double* RES) {
@@ -418,13 +449,21 @@ __global__ __launch_bounds__(64) void k_ts212(DevBasis B, DevTensor T, const TPh
         }
       }
     }
+    unsigned again = 0;
 #pragma unroll
     for (int o = 0; o < kTsOut; ++o)
       if (ob + o < p.no && lane < p.nq) {
         const TPh t = tasks[mine.y + ob + o];
-        RES[t.off] += acc[o] * (sqrt(((t.jj & 0xffff) + 1.0) * ((t.jj >> 16) + 1.0) / (1.0 + eqb) / (1.0 + eqk)) *
-                                m1pow(rank / 2));
+        if (isfinite(acc[o]))
+          RES[t.off] += acc[o] * (sqrt(((t.jj & 0xffff) + 1.0) * ((t.jj >> 16) + 1.0) / (1.0 + eqb) / (1.0 + eqk)) *
+                                  m1pow(rank / 2));
+        else
+          again |= 1u << o;
       }
+    for (; again; again &= again - 1) {
+      const TPh t = tasks[mine.y + ob + __builtin_ctz(again)];
+      RES[t.off] += ts212(B, T, t, L, Lh, R, Rh);
+    }
   }
 }
 
@@ -505,6 +544,8 @@ __global__ __launch_bounds__(64) void k_ts_ph(DevBasis B, DevTensor T, const TPh
     for (int o = 0; o < kTsOut; ++o)
       if (ob + o < p.no && lane < p.nq) {
         const TPh t = tasks[mine.y + ob + o];
+        // zero for equal orbits at odd J (2J / 2): its coefficients are zero, not its products
+        if ((eqb && ((t.jj >> 1) & 1)) || (eqk && ((t.jj >> 17) & 1))) continue;
         double sm = acc[o] * sqrt(((t.jj & 0xffff) + 1.0) * ((t.jj >> 16) + 1.0));
         if (eqb) sm *= 1.4142135623730951;
         if (eqk) sm *= 1.4142135623730951;
@@ -521,29 +562,7 @@ __global__ __launch_bounds__(256) void k_ts212_out(DevBasis B, DevTensor T, cons
   const i64 e = (i64)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= nt) return;
   const TPh t = tasks[e];
-  const int rank = T.rank, nr = rank + 1, J1 = t.jj & 0xffff, J2 = t.jj >> 16;
-  const int a = t.abcd & 255, b = (t.abcd >> 8) & 255, c = (t.abcd >> 16) & 255, d = (t.abcd >> 24) & 255;
-  const int ja = B.jj[a], jb = B.jj[b], jc = B.jj[c], jd = B.jj[d];
-  double s1 = 0.0, s2 = 0.0, s3 = 0.0, s4 = 0.0;
-  for (int k = T.fst[a * nr]; k < T.fst[(a + 1) * nr]; ++k) {
-    const int i = T.fmem[k];
-    s1 = s1 - x6(T, J1, J2, B.jj[i], ja, jb) * f_tensor_elem(B, R, Rh, a, i) * v_elem(B, L, Lh, i, b, c, d, J2);
-  }
-  for (int k = T.fst[b * nr]; k < T.fst[(b + 1) * nr]; ++k) {
-    const int i = T.fmem[k];
-    s2 = s2 + x6(T, J1, J2, B.jj[i], jb, ja) * f_tensor_elem(B, R, Rh, b, i) * v_elem(B, L, Lh, i, a, c, d, J2);
-  }
-  for (int k = T.fst[d * nr]; k < T.fst[(d + 1) * nr]; ++k) {
-    const int i = T.fmem[k];
-    s3 = s3 + x6(T, J1, J2, jd, B.jj[i], jc) * f_tensor_elem(B, R, Rh, i, d) * v_elem(B, L, Lh, a, b, c, i, J1);
-  }
-  for (int k = T.fst[c * nr]; k < T.fst[(c + 1) * nr]; ++k) {
-    const int i = T.fmem[k];
-    s4 = s4 - x6(T, J1, J2, jc, B.jj[i], jd) * f_tensor_elem(B, R, Rh, i, c) * v_elem(B, L, Lh, a, b, d, i, J1);
-  }
-  const double sm = s1 * m1pow((ja + jb - J2) / 2) + s2 * m1pow((J1 + J2) / 2) + s3 * m1pow((jc + jd - J1) / 2) +
-                    s4 * m1pow((J2 + J1) / 2);
-  RES[t.off] += sm * sqrt((J1 + 1.0) * (J2 + 1.0) / (1.0 + (a == b)) / (1.0 + (c == d))) * m1pow(rank / 2);
+  RES[t.off] += ts212(B, T, t, L, Lh, R, Rh);
 }
 
 __global__ __launch_bounds__(256) void k_ts_ph_out(DevBasis B, DevTensor T, const TPh* tasks, i64 nt, int Lh, int Rh,

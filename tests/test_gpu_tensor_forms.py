@@ -1,6 +1,7 @@
 """The two forms of the tensor terms 212 and 222_ph, one thread per output and
 one wave per pack of alike orbit quadruples: which one a tensor's size
 selects, and each against the oracle."""
+import numpy as np
 import pytest
 import torch
 
@@ -65,3 +66,32 @@ def test_form_is_set_before_the_first_use():
     tensor.TS_commutator_212(SqOp.zeros(b, -1), tensor.TensorOp.zeros(tl, 1), tensor.TensorOp.zeros(tl, 1))
     with pytest.raises(_lib.ImsrgError):
         tl.set_form("outputs")
+
+
+@pytest.mark.parametrize("emax,rank,dpar", [(2, 2, 2), (4, 4, 0), (3, 8, 0)])
+def test_nonfinite_elements_reach_the_same_outputs(emax, rank, dpar):
+    """an infinite element of L, R or a cross-coupled set reaches the outputs whose
+    sums hold it and no other, in both forms"""
+    b, _, _, tl, L, R, _ = _case(emax, rank, dpar, -1, 1, seed=9)
+    two = b.off_fpp + b.npart ** 2
+    rng = np.random.default_rng(emax)
+    spread = [0, 0]
+    for at in [two + int(x) for x in rng.integers(0, b.oplen - two, 6)] + [b.off_fph, b.off_fpp + 1]:
+        out = []
+        for form in ("outputs", "packs"):
+            t = tensor.TensorLayout(b, rank, dpar)
+            t.set_form(form)
+            L2, R2 = L.copy(), R.copy()
+            (L2 if at >= two else R2)[at] = np.inf
+            X = tensor.TensorOp.zeros(t, 1)
+            tensor.TS_commutator_212(SqOp.from_numpy(b, L2, -1), tensor.TensorOp.from_numpy(t, R2, 1), X)
+            LCC, RCC, Y = CCMat(b, -1), tensor.TensorCC(t), tensor.TensorOp.zeros(t, 1)
+            cm.calculate_cross_coupled(SqOp.from_numpy(b, L, -1), LCC)
+            LCC.data[at * 7919 % b.cclen] = float("inf")
+            tensor.TS_commutator_222_ph(LCC, RCC, tensor.TensorOp.from_numpy(t, R, 1), Y)
+            out.append([np.isfinite(Z.numpy()) for Z in (X, Y)])
+        print(f"[tensor forms] eMax {emax} rank {rank} inf at {at}", [int((~m).sum()) for o in out for m in o], flush=True)
+        for k, what in enumerate(("212", "222_ph")):
+            assert np.array_equal(out[0][k], out[1][k]), f"{what}, element {at}"
+            spread[k] += int((~out[0][k]).sum())
+    assert spread[0] > 0 and spread[1] > 0
