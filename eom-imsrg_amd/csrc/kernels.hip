@@ -166,6 +166,9 @@ void launch_comm122p(const DevBasis& B, const SegTask* t, int nt, const Partner*
 // elements of (column, row) follow from RES(c, r) = -Lh Rh RES(r, c) and are
 // written through LDS along the columns, so both orientations are stored in
 // contiguous runs.  mirror = 0: only the upper triangles of the square blocks.
+// mirror = 1: the lower triangles as well, always RESh times the upper element
+// (a diagonal tile sums both, in another order, so it mirrors its upper ones
+// through LDS too: 40Ca at eMax 8 88.7 us, 85.8 with its own lower sums stored).
 // The list kernel above is bound by the address path (about 42 vector loads an
 // element); here an element costs two loads, one store and about 30 LDS reads.
 // What bounds it now is the chain of a tile (entries, records, coefficients,
@@ -352,14 +355,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NJ <= 8 ? 4
       const int ce = __builtin_amdgcn_readlane(ce_l, c), p0 = __builtin_amdgcn_readlane(p0_l, c);
       const int cc = ce >> 28, ic = ce & 0xfffffff;
       // kept: every class pair below the diagonal, the upper triangle and,
-      // with mirror, the lower one of the square blocks
-      if (rok && (rcls < cc || (rcls == cc && (mirror || ridx <= ic))))
+      // with mirror, the lower one of the square blocks (of a diagonal tile
+      // below, as the mirror image of its own upper elements)
+      if (rok && (rcls < cc || (rcls == cc && ((mirror && !t.diag) || ridx <= ic))))
         RES[at(cc, ic, p0)] =
             rcls < cc || ridx < ic ? val[j] : (ridx == ic ? (mirror ? val[j] * RESh : val[j]) : val[j] * (hnat * RESh));
     }
   }
-  if (t.diag) return;
-  // the other orientation, through LDS: lanes along the columns
+  if (t.diag && !mirror) return;
+  // the other orientation, through LDS: lanes along the columns.  A diagonal
+  // tile holds both orientations of its rectangular elements itself.
   __syncthreads();
   {
 #pragma unroll
@@ -372,7 +377,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NJ <= 8 ? 4
     for (int r = wave; r < nrow; r += 4) {
       const int er = __builtin_amdgcn_readlane(re, r);
       const int kr = er >> 28, ir = er & 0xfffffff;
-      if (cok && (ccls_l < kr || (ccls_l == kr && (mirror || cidx_l < ir)))) {
+      if (cok && (ccls_l < kr ? !t.diag : ccls_l == kr && (t.diag ? cidx_l > ir : (mirror || cidx_l < ir)))) {
         const double v = tL[lane * LD + r];
         RES[atc(kr, ir)] = v * (ccls_l < kr || cidx_l < ir ? hnat : RESh);
       }
