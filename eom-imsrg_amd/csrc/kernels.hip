@@ -1022,6 +1022,9 @@ __device__ __forceinline__ void onebody_update(const DevBasis& B, const OneTask&
 // (p, q); its threads take the (particle a, hole i, J) terms, with (a, i)
 // from the list of particle-hole pairs inside one (l, j, tz) block (the
 // only pairs the reference's loop keeps), tree-reduced in LDS.
+// Its terms go round kOneLanes lanes; a workgroup has that many threads or half
+// of them with two lanes each (onebody_threads), and the sums are the same.
+constexpr int kOneLanes = 512;
 __device__ __forceinline__ void d_comm121(DevBasis B, const OneTask* tasks, const double* L, int Lh,
                                           const double* R, int Rh, double* RES, int RESh, int bx, double* red) {
   int inst;
@@ -1034,36 +1037,50 @@ __device__ __forceinline__ void d_comm121(DevBasis B, const OneTask* tasks, cons
   const double* Lph = L + B.off_fph;
   const double* Rph = R + B.off_fph;
   const int JS = B.jsmax;
-  double v = 0.0;
-  for (int x = threadIdx.x; x < B.nphp * JS; x += blockDim.x) {
-    const int pr = x / JS, js = x % JS;
-    const int a = B.php[2 * pr], i = B.php[2 * pr + 1];
-    const int ak = B.parts[a], ik = B.holes[i];
-    const int ji = B.jj[ik];
-    const int JT = abs(ji - jq) + 2 * js;
-    if (JT > ji + jq) continue;
-    const VPos p1 = vpos(B, ak, pk, ik, qk, JT);
-    const VPos p2 = vpos(B, ik, pk, ak, qk, JT);
-    const double la = Lph[a + (i64)i * B.P], ra = Rph[a + (i64)i * B.P];
-    v = v + (JT + 1) * (la * (Lh * vat(p1, R, Rh) - vat(p2, R, Rh)) - ra * (Rh * vat(p1, L, Lh) - vat(p2, L, Lh)));
+  double sum = 0.0;
+  for (int ln = threadIdx.x; ln < kOneLanes; ln += blockDim.x) {
+    double v = 0.0;
+    for (int x = ln; x < B.nphp * JS; x += kOneLanes) {
+      const int pr = x / JS, js = x % JS;
+      const int a = B.php[2 * pr], i = B.php[2 * pr + 1];
+      const int ak = B.parts[a], ik = B.holes[i];
+      const int ji = B.jj[ik];
+      const int JT = abs(ji - jq) + 2 * js;
+      if (JT > ji + jq) continue;
+      const VPos p1 = vpos(B, ak, pk, ik, qk, JT);
+      const VPos p2 = vpos(B, ik, pk, ak, qk, JT);
+      const double la = Lph[a + (i64)i * B.P], ra = Rph[a + (i64)i * B.P];
+      v = v + (JT + 1) * (la * (Lh * vat(p1, R, Rh) - vat(p2, R, Rh)) - ra * (Rh * vat(p1, L, Lh) - vat(p2, L, Lh)));
+    }
+    sum += v;
   }
-  const double sm = block_sum(v, red);
+  const double sm = block_sum(sum, red);
   if (threadIdx.x == 0) onebody_update(B, t, sm / (B.jj[pk] + 1.0), RES, RESh);
 }
 
-// 512 threads here and in k_comm221: a thread's items run one after the other,
-// each a chain of dependent reads (111, 121 and 221 with 256 / 512 threads: eMax
-// 6 28.0 / 24.0 us, 8 45.4 / 33.1, 10 71.7 / 54.3).
+// Threads of a workgroup of 121 and 221, n terms a result.  A thread's terms run
+// one after the other, each a chain of dependent reads, so one lane a thread is
+// faster while the launch is one round of workgroups (four of 512 threads a CU,
+// 1024 in all) and there are terms for the second half; beyond, idle threads
+// hold the place of the next results.  256 / 512 threads, us, 121 and 221: eMax 8 16O
+// (190 results) 9.4 / 7.1 and 30.1 / 20.6, four instances 13.3 / 10.9 and 48.6 / 33.6,
+// eight 16.4 / 22.6 and 58.2 / 68.7; eMax 10 (322) 13.1 / 10.3 and 46.1 / 30.0, four
+// 21.9 / 30.3 and 81.3 / 83.5; eMax 6 (100; 121 has 196 terms) 64 instances 40.6 / 71.2
+// and 119 / 150, eight 9.0 / 14.2 and 27.0 / 24.3.
+static int onebody_threads(const DevBasis& B, int nt, int n) {
+  return n > kOneLanes / 2 && (i64)nt * B.ninst <= 1024 ? kOneLanes : kOneLanes / 2;
+}
+
 __global__ __launch_bounds__(512) void k_comm121(DevBasis B, const OneTask* tasks, const double* L, int Lh,
                                                  const double* R, int Rh, double* RES, int RESh) {
-  __shared__ double red[512];
+  __shared__ double red[kOneLanes];
   d_comm121(B, tasks, L, Lh, R, Rh, RES, RESh, blockIdx.x, red);
 }
 
 void launch_comm121(const DevBasis& B, const OneTask* t, int nt, const double* L, int Lh, const double* R,
                     int Rh, double* RES, int RESh, hipStream_t s) {
   if (nt <= 0) return;
-  hipLaunchKernelGGL(k_comm121, dim3(nt, B.ninst), dim3(512), 0, s, B, t, L, Lh, R, Rh, RES, RESh);
+  hipLaunchKernelGGL(k_comm121, dim3(nt, B.ninst), dim3(onebody_threads(B, nt, B.nphp * B.jsmax)), 0, s, B, t, L, Lh, R, Rh, RES, RESh);
 }
 
 // ============================================================ commutator_221
@@ -1103,44 +1120,48 @@ __device__ __forceinline__ void d_comm221(DevBasis B, const OneTask* tasks, cons
   const int pm = Lh * Rh;
   const bool both = (t.kind != 2);
   const int JS = B.jsmax;
-  double v = 0.0;
-  // thread item (c, J): intermediate orbit c (holes first, with w1; then
-  // particles, with w2) and one 2J of its coupling to i
-  for (int y = threadIdx.x; y < B.N * JS; y += blockDim.x) {
-    const int x = y / JS;
-    const bool hole = x < B.A;
-    const int ck = hole ? B.holes[x] : B.parts[x - B.A];
-    const int jc = B.jj[ck];
-    const int JT = abs(jc - ji) + 2 * (y % JS);
-    if (JT > jc + ji) continue;
-    if (hole) {
-      if (both)
-        v = v + (v_elem(B, w1, 1, ck, ik, ck, jk, JT) - pm * v_elem(B, w1, 1, ck, jk, ck, ik, JT)) * (JT + 1);
-      else
-        v = v + v_elem(B, w1, 1, ck, ik, ck, jk, JT) * (JT + 1);
-    } else {
-      if (both)
-        v = v + (w2_elem(B, w2, L, R, Rh, ck, ik, ck, jk, JT) - pm * w2_elem(B, w2, L, R, Rh, ck, jk, ck, ik, JT)) *
-                    (JT + 1);
-      else
-        v = v + w2_elem(B, w2, L, R, Rh, ck, ik, ck, jk, JT) * (JT + 1);
+  double sum = 0.0;
+  // item (c, J): intermediate orbit c (holes first, with w1; then particles,
+  // with w2) and one 2J of its coupling to i
+  for (int ln = threadIdx.x; ln < kOneLanes; ln += blockDim.x) {
+    double v = 0.0;
+    for (int y = ln; y < B.N * JS; y += kOneLanes) {
+      const int x = y / JS;
+      const bool hole = x < B.A;
+      const int ck = hole ? B.holes[x] : B.parts[x - B.A];
+      const int jc = B.jj[ck];
+      const int JT = abs(jc - ji) + 2 * (y % JS);
+      if (JT > jc + ji) continue;
+      if (hole) {
+        if (both)
+          v = v + (v_elem(B, w1, 1, ck, ik, ck, jk, JT) - pm * v_elem(B, w1, 1, ck, jk, ck, ik, JT)) * (JT + 1);
+        else
+          v = v + v_elem(B, w1, 1, ck, ik, ck, jk, JT) * (JT + 1);
+      } else {
+        if (both)
+          v = v + (w2_elem(B, w2, L, R, Rh, ck, ik, ck, jk, JT) - pm * w2_elem(B, w2, L, R, Rh, ck, jk, ck, ik, JT)) *
+                      (JT + 1);
+        else
+          v = v + w2_elem(B, w2, L, R, Rh, ck, ik, ck, jk, JT) * (JT + 1);
+      }
     }
+    sum += v;
   }
-  const double sm = block_sum(v, red);
+  const double sm = block_sum(sum, red);
   if (threadIdx.x == 0) onebody_update(B, t, sm / (ji + 1.0), RES, RESh);
 }
 
 __global__ __launch_bounds__(512) void k_comm221(DevBasis B, const OneTask* tasks, const double* L, int Lh,
                                                  const double* R, int Rh, const double* w1, const double* w2,
                                                  double* RES, int RESh) {
-  __shared__ double red[512];
+  __shared__ double red[kOneLanes];
   d_comm221(B, tasks, L, Lh, R, Rh, w1, w2, RES, RESh, blockIdx.x, red);
 }
 
 void launch_comm221(const DevBasis& B, const OneTask* t, int nt, const double* L, int Lh, const double* R, int Rh,
                     const double* w1, const double* w2, double* RES, int RESh, hipStream_t s) {
   if (nt <= 0) return;
-  hipLaunchKernelGGL(k_comm221, dim3(nt, B.ninst), dim3(512), 0, s, B, t, L, Lh, R, Rh, w1, w2, RES, RESh);
+  hipLaunchKernelGGL(k_comm221, dim3(nt, B.ninst), dim3(onebody_threads(B, nt, B.N * B.jsmax)), 0, s, B, t, L, Lh, R, Rh, w1, w2, RES, RESh);
 }
 
 // ================================================= commutator_110 + 220 (E0)
@@ -2047,7 +2068,7 @@ __global__ __launch_bounds__(256) void k_phase2(DevBasis B, Phase2 P) {
 
 // 121 and 221 of a one-body element in its workgroup, in that order
 __global__ __launch_bounds__(512) void k_phase3(DevBasis B, Phase3 P) {
-  __shared__ union { PhChunkLds c; double red[512]; } lds;
+  __shared__ union { PhChunkLds c; double red[kOneLanes]; } lds;
   int inst;
   if (!batch_inst(B, inst)) return;
   int b = blockIdx.x;
