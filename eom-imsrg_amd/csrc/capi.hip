@@ -1233,13 +1233,26 @@ void t_tail(const Exec& X, double* RES, int RESh, const Append* ap, hipStream_t 
 }
 
 // The small bases whose commutator runs in three launches: every family on
-// 32 x 32 LDS tiles with its usual transposes, 122 by lists, 222_ph by chunks
-bool small_phases(const Exec& X) {
-  imsrg_basis_s* B = X.B;
+// 32 x 32 LDS tiles with its usual transposes, 122 by lists, 222_ph by chunks.
+// Most instances of one call in that form: with more workgroups than kPhaseGroups
+// the terms fill the chip by themselves, and the shared launches, which take the
+// registers and LDS of their largest term, lose.  Three launches / a launch per
+// term, us: eMax 4 16O (1604 workgroups an instance) 1 instance 58 / 136, 8 138 / 160,
+// 16 231 / 213, 64 812 / 600; eMax 3 (739) 16 116 / 148, 32 184 / 178; eMax 2 4He (356)
+// 64 150 / 159, 128 269 / 216; eMax 6 lMax 3 (3679) 4 166 / 176, 8 286 / 251; BCH by
+// graphs turns a little later (eMax 4 16 instances 3331 / 3231, eMax 3 32 2468 / 2655).
+constexpr int kPhaseGroups = 18000;
+int phase_instances(const imsrg_basis_s* B) {
   auto fits = [](const GemmFamily& f, int sig) { return f.tasks.n == 0 || (f.tile == 5 && f.sig == sig); };
-  return B->path == IMSRG_PATH_GROUPED && !B->t122_ok && !B->phb_ok && fits(B->pp1, 8) && fits(B->k2, 0) &&
-         fits(B->k3, 1) && fits(B->ph, 10);
+  if (!B->dev_ready || B->path != IMSRG_PATH_GROUPED || B->t122_ok || B->phb_ok || !fits(B->pp1, 8) ||
+      !fits(B->k2, 0) || !fits(B->k3, 1) || !fits(B->ph, 10))
+    return 0;
+  int n = B->seg_tri.n + B->cc.n + B->pairs.n + B->seg_epi.n + (int)B->one_h.size() + (int)B->phc_h.size() +
+          (int)(((i64)B->b.A * B->b.A + (i64)B->b.P * B->b.A + (i64)B->b.P * B->b.P) / 4);
+  for (const GemmFamily* f : {&B->pp1, &B->k2, &B->k3, &B->ph}) n += f->tasks.n;
+  return kPhaseGroups / std::max(n, 1);
 }
+bool small_phases(const Exec& X) { return X.D.ninst <= phase_instances(X.B); }
 PhaseGemm phase_gemm(const Exec& X, const GemmFamily& f, const double* a, const double* b, const double* c, i64 st,
                      i64 sc, double as = 1.0, double s2 = 1.0) {
   PhaseGemm g{};
@@ -2751,6 +2764,7 @@ int64_t imsrg_basis_size(imsrg_basis B, int what) {
         n += (i64)(b.spstart[q + 1] - b.spstart[q]) * (b.spstart[q + 1] - b.spstart[q]);
       return n;
     }
+    case IMSRG_SIZE_PHASES: return phase_instances(B);
   }
   return -1;
 }

@@ -24,7 +24,8 @@ IMSRG_ECLIP = 3
 IMSRG_ESTEPS = 4
 PATH_GROUPED = 0
 PATH_PLAIN = 1
-SIZE = dict(NORB=0, NHOLE=1, NPART=2, JTOTAL_MAX=3, NBLOCKS=4, OP=5, NCC=6, CC=7, WCC=8, NEQ=9, SPMAT=10)
+SIZE = dict(NORB=0, NHOLE=1, NPART=2, JTOTAL_MAX=3, NBLOCKS=4, OP=5, NCC=6, CC=7, WCC=8, NEQ=9, SPMAT=10,
+            PHASES=11)
 
 
 class ImsrgError(RuntimeError):

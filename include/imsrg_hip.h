@@ -59,6 +59,7 @@ typedef void* imsrg_stream;
 #define IMSRG_SIZE_WCC 8  /* doubles of the WCC workspace */
 #define IMSRG_SIZE_NEQ 9  /* doubles of the vectorize stream (H%neq) */
 #define IMSRG_SIZE_SPMAT 10 /* doubles of a single-particle block matrix set (full_sp_block_mat) */
+#define IMSRG_SIZE_PHASES 11 /* most instances whose fused commutator takes three launches (0 before the first call) */
 
 const char* imsrg_last_error(void);
 
