@@ -393,50 +393,64 @@ void build_t122(imsrg_basis_s* B, const std::vector<int>& order) {
   struct Set { int a, b; std::vector<int> ent; };   // one pair of (l, j, tz) blocks
   struct Group { int row0, nrow; std::vector<std::pair<int, int>> slab; };   // (col0, ncol)
   std::vector<std::vector<Set>> sets(b.nblocks);
-  int big = 0;
+  int big = 0, most = 0;   // largest closed set; most pairs of a channel's class
+  const int nb = (int)b.spstart.size() - 1;
+  std::vector<std::vector<int>> m((size_t)nb * nb);
   for (int q = 0; q < b.nblocks; ++q) {
-    std::map<std::pair<int, int>, std::vector<int>> m;
-    for (int c = 0; c < 3; ++c)
+    for (int c = 0; c < 3; ++c) {
+      const std::vector<int>& pl = b.pl[q * 3 + c];
+      most = std::max(most, b.dims[q * 3 + c]);
       for (int ix = 0; ix < b.dims[q * 3 + c]; ++ix) {
-        const int x = b.spblk[b.pl[q * 3 + c][2 * ix]], y = b.spblk[b.pl[q * 3 + c][2 * ix + 1]];
-        m[{std::min(x, y), std::max(x, y)}].push_back((c << 28) | ix);
+        const int x = b.spblk[pl[2 * ix]], y = b.spblk[pl[2 * ix + 1]];
+        m[(size_t)std::min(x, y) * nb + std::max(x, y)].push_back((c << 28) | ix);
       }
-    for (auto& kv : m) {
-      big = std::max(big, (int)kv.second.size());
-      sets[q].push_back(Set{kv.first.first, kv.first.second, std::move(kv.second)});
     }
+    for (int x = 0; x < nb; ++x)
+      for (int y = x; y < nb; ++y) {
+        std::vector<int>& e = m[(size_t)x * nb + y];
+        if (e.empty()) continue;
+        big = std::max(big, (int)e.size());
+        sets[q].push_back(Set{x, y, std::move(e)});
+        e.clear();
+      }
   }
   // slabs as wide as the kernels' unrolled column counts
   if (big > kT122Cols) return;
   const int cap = big <= 16 ? 16 : (big <= 32 ? 32 : (big <= 40 ? 40 : kT122Cols));
+  // place of a pair in the sorted entries under way, -1 elsewhere
+  std::vector<int> at((size_t)3 * most, -1);
+  auto place = [&](int c, int ix) -> int& { return at[(size_t)c * most + ix]; };
   auto emit = [&](int q, std::vector<int> ent, const std::vector<int>& ptr, std::vector<int>& out,
-                  std::vector<int>& cnt, std::vector<std::vector<int2>>& recs) {
+                  std::vector<int>& cnt, std::vector<int2>& recs) {
     std::sort(ent.begin(), ent.end());
-    std::map<int, int> at;
-    for (size_t x = 0; x < ent.size(); ++x) at[ent[x]] = (int)x;
-    for (int e : ent) {
-      const int c = e >> 28, ix = e & 0xfffffff;
+    for (size_t x = 0; x < ent.size(); ++x) place(ent[x] >> 28, ent[x] & 0xfffffff) = (int)x;
+    bool ok = true;
+    for (size_t x = 0; ok && x < ent.size(); ++x) {
+      const int c = ent[x] >> 28, ix = ent[x] & 0xfffffff;
       const size_t gid = (size_t)b.pairoff[q * 3 + c] + ix;
       const bool same = b.pl[q * 3 + c][2 * ix] == b.pl[q * 3 + c][2 * ix + 1];
-      std::vector<int2> r;
+      const int n = ptr[gid + 1] - ptr[gid];
+      if (n > kT122Recs) {
+        ok = false;
+        break;
+      }
       for (int k = ptr[gid]; k < ptr[gid + 1]; ++k) {
         const Partner& p = B->part_h[k];
-        const auto it = at.find((((p.code >> 22) & 3) << 28) | (p.code & 0x3fffff));
-        if (it == at.end()) return false;
+        const int i = place((p.code >> 22) & 3, p.code & 0x3fffff);
+        ok = ok && i >= 0;
         const int s2 = (p.code >> 26) & 1;
-        r.push_back(int2{it->second | (((p.code >> 24) & 1) << 17) | (((p.code >> 25) & 1) << 18) |
-                             ((s2 == (same ? 1 : 0) ? 0 : (s2 ? 1 : 2)) << 19),
-                         B->f1off_h[p.fk]});
+        recs.push_back(int2{i | (((p.code >> 24) & 1) << 17) | (((p.code >> 25) & 1) << 18) |
+                                ((s2 == (same ? 1 : 0) ? 0 : (s2 ? 1 : 2)) << 19),
+                            B->f1off_h[p.fk]});
       }
-      if (r.size() > (size_t)kT122Recs) return false;
-      P.maxrec = std::max(P.maxrec, (int)r.size());
-      out.push_back(e);
-      cnt.push_back((int)r.size());
-      recs.push_back(std::move(r));
+      P.maxrec = std::max(P.maxrec, n);
+      out.push_back(ent[x]);
+      cnt.push_back(n);
     }
-    return true;
+    for (int e : ent) place(e >> 28, e & 0xfffffff) = -1;
+    return ok;
   };
-  std::vector<std::vector<int2>> rr, cr;
+  std::vector<int2> rr, cr;   // the records of the entries one after the other
   for (int q : order) {
     std::vector<Group> gs;
     size_t x = 0;
@@ -473,15 +487,17 @@ void build_t122(imsrg_basis_s* B, const std::vector<int>& order) {
   P.nrows = (int)B->t122_rent.size();
   P.ncols = (int)B->t122_cent.size();
   if (P.maxrec < 1) P.maxrec = 1;
-  auto flat = [](const std::vector<std::vector<int2>>& v, int maxrec, std::vector<int2>& out) {
-    out.assign((size_t)maxrec * v.size(), int2{0, 0});
-    for (size_t i = 0; i < v.size(); ++i)
-      for (size_t k = 0; k < v[i].size(); ++k) out[k * v.size() + i] = v[i][k];
-  };
-  flat(rr, P.maxrec, B->t122_rrec);
-  flat(cr, P.maxrec, B->t122_crec);
   B->t122t.n = (int)B->t122t.host.size();
   B->t122_ok = B->t122t.n >= kT122MinTiles;
+  if (!B->t122_ok) return;
+  auto flat = [&](const std::vector<int2>& v, const std::vector<int>& cnt, std::vector<int2>& out) {
+    out.assign((size_t)P.maxrec * cnt.size(), int2{0, 0});
+    size_t at = 0;
+    for (size_t i = 0; i < cnt.size(); ++i)
+      for (int k = 0; k < cnt[i]; ++k) out[(size_t)k * cnt.size() + i] = v[at++];
+  };
+  flat(rr, B->t122_rcnt, B->t122_rrec);
+  flat(cr, B->t122_ccnt, B->t122_crec);
 }
 
 // 222_ph by block quadruples: the cross-coupled rows in block order, the
