@@ -410,7 +410,8 @@ __global__ __launch_bounds__(64) void k_ts212(DevBasis B, DevTensor T, const TPh
             double c = 0.0;
             if (o < p.no) {
               const int jj = tasks[f0 + o].jj, J1 = jj & 0xffff, J2 = jj >> 16;
-              if ((bra ? J2 : J1) == J) {
+              // the two terms of a pair of equal orbits cancel at odd J (2J / 2)
+              if ((bra ? J2 : J1) == J && !(bra ? eqb && ((J1 >> 1) & 1) : eqk && ((J2 >> 1) & 1))) {
                 if (sd == 0) c = -x6(T, J1, J2, ji, jx, jy) * m1pow((jx + jy - J2) / 2);
                 else if (sd == 1) c = x6(T, J1, J2, ji, jx, jy) * m1pow((J1 + J2) / 2);
                 else if (sd == 2) c = x6(T, J1, J2, jx, ji, jy) * m1pow((jx + jy - J1) / 2);

@@ -95,3 +95,29 @@ def test_nonfinite_elements_reach_the_same_outputs(emax, rank, dpar):
             assert np.array_equal(out[0][k], out[1][k]), f"{what}, element {at}"
             spread[k] += int((~out[0][k]).sum())
     assert spread[0] > 0 and spread[1] > 0
+
+
+@pytest.mark.parametrize("emax,rank,dpar", [(2, 2, 2), (4, 4, 0), (3, 8, 0)])
+def test_forbidden_elements_stay_zero(emax, rank, dpar):
+    """two equal orbits do not couple to odd J: where one thread per output leaves
+    such an element exactly zero, so do the packs"""
+    b, _, _, tl, L, R, _ = _case(emax, rank, dpar, -1, 1, seed=13)
+    zero = []
+    for form in ("outputs", "packs"):
+        t = tensor.TensorLayout(b, rank, dpar)
+        t.set_form(form)
+        Ld, Rd = SqOp.from_numpy(b, L, -1), tensor.TensorOp.from_numpy(t, R, 1)
+        X, Y = tensor.TensorOp.zeros(t, 1), tensor.TensorOp.zeros(t, 1)
+        tensor.TS_commutator_212(Ld, Rd, X)
+        LCC, RCC = CCMat(b, -1), tensor.TensorCC(t)
+        cm.calculate_cross_coupled(Ld, LCC)
+        tensor.TS_commutator_222_ph(LCC, RCC, Rd, Y)
+        zero.append([Z.numpy() == 0.0 for Z in (X, Y)])
+    odd = np.zeros(tl.oplen, bool)
+    for q, g, ix, jx, (a, c), (d, e), J1, J2, at in tl.elements():
+        odd[at] = (a == c and J1 // 2 % 2 == 1) or (d == e and J2 // 2 % 2 == 1)
+    print(f"[tensor forms] eMax {emax} rank {rank}: {int(odd.sum())} forbidden, zero by form",
+          [[int(z[odd].sum()) for z in f] for f in zero], flush=True)
+    for k, what in enumerate(("212", "222_ph")):
+        assert odd.any() and zero[0][k][odd].any()
+        assert not (zero[0][k] & odd & ~zero[1][k]).any(), what
