@@ -166,9 +166,10 @@ void launch_comm122p(const DevBasis& B, const SegTask* t, int nt, const Partner*
 // elements of (column, row) follow from RES(c, r) = -Lh Rh RES(r, c) and are
 // written through LDS along the columns, so both orientations are stored in
 // contiguous runs.  mirror = 0: only the upper triangles of the square blocks.
-// mirror = 1: the lower triangles as well, always RESh times the upper element
-// (a diagonal tile sums both, in another order, so it mirrors its upper ones
-// through LDS too: 40Ca at eMax 8 88.7 us, 85.8 with its own lower sums stored).
+// mirror = 1: the lower triangles as well, always RESh times the upper element.
+// A diagonal tile sums both, in another order, so it stores its upper ones twice,
+// the image in scattered single elements: eMax 6 16.4 us, 7 34.0, 8 70.3 (with its
+// own lower sums, in runs, 16.3, 33.5, 69.4; the image through LDS 17.8, 36.4, 72.7).
 // The list kernel above is bound by the address path (about 42 vector loads an
 // element); here an element costs two loads, one store and about 30 LDS reads.
 // What bounds it now is the chain of a tile (entries, records, coefficients,
@@ -356,15 +357,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NJ <= 8 ? 4
       const int cc = ce >> 28, ic = ce & 0xfffffff;
       // kept: every class pair below the diagonal, the upper triangle and,
       // with mirror, the lower one of the square blocks (of a diagonal tile
-      // below, as the mirror image of its own upper elements)
+      // the mirror image of its own upper elements)
       if (rok && (rcls < cc || (rcls == cc && ((mirror && !t.diag) || ridx <= ic))))
         RES[at(cc, ic, p0)] =
             rcls < cc || ridx < ic ? val[j] : (ridx == ic ? (mirror ? val[j] * RESh : val[j]) : val[j] * (hnat * RESh));
+      if (t.diag && mirror && rok && rcls == cc && ridx < ic)   // row ic, column ridx
+        RES[at(cc, ridx, p0 - ic + ridx) + (ic - ridx)] = val[j] * RESh;
     }
   }
-  if (t.diag && !mirror) return;
-  // the other orientation, through LDS: lanes along the columns.  A diagonal
-  // tile holds both orientations of its rectangular elements itself.
+  if (t.diag) return;
+  // the other orientation, through LDS: lanes along the columns
   __syncthreads();
   {
 #pragma unroll
@@ -377,7 +379,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NJ <= 8 ? 4
     for (int r = wave; r < nrow; r += 4) {
       const int er = __builtin_amdgcn_readlane(re, r);
       const int kr = er >> 28, ir = er & 0xfffffff;
-      if (cok && (ccls_l < kr ? !t.diag : ccls_l == kr && (t.diag ? cidx_l > ir : (mirror || cidx_l < ir)))) {
+      if (cok && (ccls_l < kr || (ccls_l == kr && (mirror || cidx_l < ir)))) {
         const double v = tL[lane * LD + r];
         RES[atc(kr, ir)] = v * (ccls_l < kr || cidx_l < ir ? hnat : RESh);
       }
