@@ -695,8 +695,9 @@ void launch_comm222ph_chunk(const DevBasis& B, const PhChunk* ch, int nch, const
 // lines: the address path was busy 90 % of its time, 1.09 GB a launch at eMax 8
 // for 0.41 GB of data); here the lanes run along rows of n_A n_C elements and
 // neighbouring waves share what is left of a line (0.40 GB).  Bound now by
-// vector instructions (index arithmetic: 62 % of the time at eight waves a
-// SIMD).  eMax 7 / 8 / 10: 69 / 182 / 1199 -> 46 / 93 / 642 us.  Tried: one
+// vector instructions (index arithmetic: the vector units issue 60 % of the
+// time with 16 waves a CU, on average over a launch, of the 29 that 5.6 KB of
+// LDS each let in).  eMax 7 / 8 / 10: 69 / 182 / 1199 -> 46 / 93 / 642 us.  Tried: one
 // workgroup per 3072 values of several quadruples, searched per lane (194 us at
 // eMax 8, 3200 vector instructions a wave); a wave per quadruple in workgroups
 // of four with 1024 values each (151 us: half the occupancy).
