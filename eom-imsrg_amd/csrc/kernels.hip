@@ -169,7 +169,7 @@ void launch_comm122p(const DevBasis& B, const SegTask* t, int nt, const Partner*
 // mirror = 1: the lower triangles as well, always RESh times the upper element.
 // A diagonal tile sums both, in another order, so it stores its upper ones twice,
 // the image in scattered single elements: eMax 6 16.4 us, 7 34.0, 8 70.3 (with its
-// own lower sums, in runs, 16.3, 33.5, 69.4; the image through LDS 17.8, 36.4, 72.7).
+// own lower sums, in runs, 16.5, 33.9, 69.3; the image through LDS 17.8, 36.4, 72.7).
 // The list kernel above is bound by the address path (about 42 vector loads an
 // element); here an element costs two loads, one store and about 30 LDS reads.
 // What bounds it now is the chain of a tile (entries, records, coefficients,
@@ -349,6 +349,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NJ <= 8 ? 4
     }
   }
   // outputs stored as (r, c)
+  const bool lower = mirror && !t.diag;
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
     const int c = wave + 4 * j;
@@ -356,16 +357,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NJ <= 8 ? 4
       const int ce = __builtin_amdgcn_readlane(ce_l, c), p0 = __builtin_amdgcn_readlane(p0_l, c);
       const int cc = ce >> 28, ic = ce & 0xfffffff;
       // kept: every class pair below the diagonal, the upper triangle and,
-      // with mirror, the lower one of the square blocks (of a diagonal tile
-      // the mirror image of its own upper elements)
-      if (rok && (rcls < cc || (rcls == cc && ((mirror && !t.diag) || ridx <= ic))))
+      // with mirror, the lower one of the square blocks
+      if (rok && (rcls < cc || (rcls == cc && (lower || ridx <= ic))))
         RES[at(cc, ic, p0)] =
             rcls < cc || ridx < ic ? val[j] : (ridx == ic ? (mirror ? val[j] * RESh : val[j]) : val[j] * (hnat * RESh));
-      if (t.diag && mirror && rok && rcls == cc && ridx < ic)   // row ic, column ridx
-        RES[at(cc, ridx, p0 - ic + ridx) + (ic - ridx)] = val[j] * RESh;
     }
   }
-  if (t.diag) return;
+  if (t.diag) {
+    if (!mirror) return;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int c = wave + 4 * j;
+      if (c < ncol) {   // row ic, column ridx
+        const int ce = __builtin_amdgcn_readlane(ce_l, c), p0 = __builtin_amdgcn_readlane(p0_l, c);
+        const int cc = ce >> 28, ic = ce & 0xfffffff;
+        if (rok && rcls == cc && ridx < ic) RES[at(cc, ridx, p0 - ic + ridx) + (ic - ridx)] = val[j] * RESh;
+      }
+    }
+    return;
+  }
   // the other orientation, through LDS: lanes along the columns
   __syncthreads();
   {
