@@ -13,7 +13,9 @@
  *
  * every block column-major exactly as the Fortran sq_op holds it
  * (basic_IMSRG.f90:50-76,619-628).  The herm flag (+1 / -1) of each operand
- * travels beside its pointer, as sq_op%herm does.  Cross-coupled matrices
+ * travels beside its pointer, as sq_op%herm does; operands are (anti)hermitian
+ * as flagged, square blocks stored in both triangles (kernels read whichever
+ * of an element and its image lies better).  Cross-coupled matrices
  * (type cc_mat) are device buffers of imsrg_basis_size(IMSRG_SIZE_CC)
  * doubles; the WCC workspace has imsrg_basis_size(IMSRG_SIZE_WCC) doubles.
  *
